@@ -16,11 +16,15 @@
 //    latency behind the serial recurrence (small grids leave only a few
 //    waves per SIMD); per-group coefficients, dose weights included, come
 //    through the scalar cache so they never queue behind the ring;
+//  * grids of few lanes share a lane between two threads, one per linear form
+//    (energy_split_kernel);
 //  * the final E-half of a depth step also accumulates the Eq.24 dose and the
 //    psi^2 proxy in FP64 (block partials, reduced deterministically later), so
 //    the IDD costs no extra pass over the state.
 
+#include "buffer.hpp"
 #include "kernels.hpp"
+#include "mfma.hpp"
 
 #include <type_traits>
 
@@ -484,6 +488,260 @@ __global__ __launch_bounds__(kBlock) void energy_pair_kernel(
     if (tops.out_x) publish_top(top_a, tops.out_x, nullptr, ldi);
 }
 
+// ------------------------------------------------------ few lanes: split ---
+// The sweeps on grids of few lanes (energy_split).  There the time is the
+// serial walk over the groups of a wave that has a SIMD to itself: the
+// instructions it issues per group and every latency it exposes.  One thread
+// per lane left most SIMDs idle and waited at every group for coefficients
+// (scalar loads return out of order, so the wait for the second half's set
+// also drained the prefetch of the next).  Here
+//  * two adjacent threads share a lane and evaluate one linear form each
+//    (role 0: f, role 1: F), exchanging results by a DPP swap: half the
+//    arithmetic per wave and twice the waves, one per work-group, so they
+//    spread over the CUs;
+//  * the coefficients of 16 groups at a time are staged in LDS in the order
+//    the roles read them; a group's are read one group ahead, and the second
+//    half's are the registers the first half used one group before;
+//  * rows are addressed through buffer resources by one running scalar offset,
+//    and the highest nonzero group is looked for only until it is found.
+// The operations on each value are those of recur(), in its order, so states
+// are bit-identical to the kernels above.  Loads and stores are temporal: at
+// these sizes the state stays in the caches between operators.
+constexpr int kSplitRing = 16;  // groups per LDS chunk, the unroll
+// Slots of the register ring (a divisor of kSplitRing).
+template <typename T, bool FOUR>
+constexpr int split_ring() { return FOUR || sizeof(T) == 8 ? 8 : 16; }
+
+// Lanes of one array from which one thread per lane is the better sweep: 2^16
+// lanes are 2048 waves here, the two per SIMD that its registers allow; one
+// more round of waves costs what the split gains.  Measured (FP32, straggling,
+// primary with its copy and secondary with two sources, mean of the two, one
+// kernel at a time): 14,641 lanes x 500 groups 207 -> 83 us, 25,600 x 500
+// 207 -> 105 us, 46,656 x 400 176 -> 104 us; 74,529 x 400 214 -> 243 us.
+constexpr long long kSplitLanes = 1LL << 16;
+inline bool energy_split(long long lanes, int Ng, size_t elem) {
+    return lanes < kSplitLanes && lanes * Ng * static_cast<long long>(elem) < (1LL << 31);
+}
+
+__device__ inline double swap_pair(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = __builtin_amdgcn_mov_dpp(static_cast<int>(u), 0xB1, 0xF, 0xF, false);
+    const unsigned hi = __builtin_amdgcn_mov_dpp(static_cast<int>(u >> 32), 0xB1, 0xF, 0xF, false);
+    return __builtin_bit_cast(double, (static_cast<unsigned long long>(hi) << 32) | lo);
+}
+__device__ inline float swap_pair(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, false));
+}
+
+// One role's coefficients of a group: the form's seven (the output
+// difference's negated for role 0, whose difference is) and its dose weight.
+struct RoleForm {
+    double c[8];
+};
+
+// One half's carried values in a thread: inputs at g + 1, and own - other of
+// its outputs there (b - a for role 1, the negation for role 0).
+template <typename T>
+struct SplitHalf {
+    double P_hi = 0.0, R_hi = 0.0, diff = 0.0;
+    // The thread's output at g: recur()'s `a` (role 0) or `b` (role 1).
+    template <bool SRC, bool STRAG>
+    __device__ inline double step(const RoleForm& k, double P, double R, double P_lo, double src) {
+        double v = fma(k.c[3], R, fma(k.c[2], P, fma(k.c[1], R_hi, k.c[0] * P_hi)));
+        if (STRAG) v = fma(k.c[4], P_lo, v);
+        if (SRC) v = fma(k.c[5], src, v);
+        v = flush_tiny<T>(fma(k.c[6], diff, v));
+        P_hi = P;
+        R_hi = R;
+        diff = v - swap_pair(v);
+        return v;
+    }
+};
+
+// PAIR: the two half steps of energy_pair_kernel (DOSE is always on then);
+// otherwise energy_half_kernel.  One wave per work-group, 32 lanes.  XOUT
+// writes every group up to the top: a branch per group costs more here than
+// the rows nobody reads.
+template <typename T, bool PAIR, bool SRC, bool STRAG, bool DOSE, bool XOUT>
+__global__ __launch_bounds__(64) void energy_split_kernel(
+    T* __restrict__ F, T* __restrict__ f, const EnergyCoef* __restrict__ coef,
+    const T* __restrict__ Qa, const T* __restrict__ Qb, T* __restrict__ XF, T* __restrict__ Xf,
+    int Ng, int lanes, const double* __restrict__ yzw, int nang, double* __restrict__ partials,
+    int proxy, SweepTops tops) {
+    typedef double f64x2 __attribute__((ext_vector_type(2)));
+    constexpr int R = kSplitRing;
+    constexpr int RING = split_ring<T, PAIR && SRC>(), D = RING - 1;
+    __shared__ __attribute__((aligned(16))) double forms[2][R][2][8];  // [chunk][group][role]
+    reset_tops(tops);
+    const int role = threadIdx.x & 1;
+    const int own_lane = blockIdx.x * 32 + (threadIdx.x >> 1);
+    // Threads past the last lane repeat it: they sit in the wave that owns it,
+    // so they load and store the same values in the same instructions.
+    const bool live = own_lane < lanes;
+    const int lane = min(own_lane, lanes - 1);
+    const int qa_top = SRC ? source_top(tops, tops.xa, Ng) : -1;
+    const int qb_top = SRC && PAIR ? source_top(tops, tops.xb, Ng) : -1;
+    const int t1 = max(state_top(tops, Ng), qa_top) + (STRAG ? 1 : 0);
+    const int G0 = min(Ng - 1, PAIR ? max(t1, qb_top) + (STRAG ? 1 : 0) : t1);
+    int top_a = -1, top_b = -1;
+    double dose = 0.0, psum = 0.0;
+    if (G0 >= 0) {
+        const int row = lanes * static_cast<int>(sizeof(T));  // bytes of one group's row
+        const unsigned bytes = static_cast<unsigned>(row) * static_cast<unsigned>(Ng);
+        const __amdgpu_buffer_rsrc_t bF = make_rsrc(F, bytes), bf = make_rsrc(f, bytes);
+        const __amdgpu_buffer_rsrc_t ba = make_rsrc(const_cast<T*>(SRC ? Qa : F), bytes);
+        const __amdgpu_buffer_rsrc_t bb = make_rsrc(const_cast<T*>(SRC && PAIR ? Qb : F), bytes);
+        const unsigned voff = static_cast<unsigned>(lane) * sizeof(T);
+        const int qa_row = max(qa_top, 0) * row, qb_row = max(qb_top, 0) * row;
+        T rF[RING], rf[RING], rQa[RING], rQb[RING];
+        auto fetch = [&](int k, int at) {  // the row at byte offset `at` into slot k
+            rF[k] = bload<T>(bF, voff, at);
+            rf[k] = bload<T>(bf, voff, at);
+            if (SRC) rQa[k] = bload<T>(ba, voff, min(at, qa_row));
+        };
+        auto fetch_qb = [&](int k, int at) {
+            if (SRC && PAIR) rQb[k] = bload<T>(bb, voff, min(at, qb_row));
+        };
+        // Chunk staging: thread t holds four values of group g0 - t / 4: role
+        // (t / 2) % 2, values 4 (t % 2) .. + 3 of that role's RoleForm.
+        const int ck = threadIdx.x >> 2, cr = (threadIdx.x >> 1) & 1, ch = threadIdx.x & 1;
+        double st[4];
+        auto stage_load = [&](int g0) {
+            const double* c = reinterpret_cast<const double*>(coef + max(g0 - ck, 0)) + 7 * cr + 4 * ch;
+#pragma unroll
+            for (int e = 0; e < 3; ++e) st[e] = c[e];
+            st[3] = c[ch && !cr ? 11 : 3];  // the weights: w1 follows aF, w2 closes the record
+        };
+        auto stage_store = [&](int buf) {
+            f64x2* dst = reinterpret_cast<f64x2*>(&forms[buf][ck][cr][4 * ch]);
+            dst[0] = f64x2{st[0], st[1]};
+            dst[1] = f64x2{ch && !cr ? -st[2] : st[2], st[3]};
+        };
+        auto read_form = [&](int buf, int k) {
+            RoleForm r;
+            const f64x2* src = reinterpret_cast<const f64x2*>(&forms[buf][k][role][0]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const f64x2 v = src[e];
+                r.c[2 * e] = v[0];
+                r.c[2 * e + 1] = v[1];
+            }
+            return r;
+        };
+        // (both before the ring's first loads, as in the steady state: the wait
+        // for a chunk's coefficients must not be a wait for the ring)
+        stage_load(G0);
+        stage_store(0);
+        stage_load(G0 - R);
+        int ld = G0 * row;  // row of the next load, clamped at group 0
+        int sto = ld;       // row of the step's group
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+            fetch(k, ld);
+            fetch_qb(k, ld);
+            ld = max(ld - row, 0);
+        }
+        wave_lds_sync();
+        SplitHalf<T> one, two;
+        double P2 = 0.0, R2 = 0.0;  // the first half's outputs at g + 1, rounded to the state type
+        char* const out = reinterpret_cast<char*>((role ? F : f) + lane);
+        char* const xout = XOUT ? reinterpret_cast<char*>((role ? XF : Xf) + lane) : nullptr;
+        RoleForm cn = read_form(0, 0), c2 = {};
+        auto put = [](char* p, int at, T v) { *reinterpret_cast<T*>(p + static_cast<unsigned>(at)) = v; };
+        // The source of a group, zero above its top (where the row is not its own).
+        auto source = [](T q, bool on) { return on ? static_cast<double>(q) : 0.0; };
+        // The second half at g2 (row at, coefficients c2).
+        auto second = [&](int g2, int at, double P_lo, T q, auto track) {
+            const double v = two.template step<SRC, STRAG>(c2, P2, R2, P_lo,
+                                                           SRC ? source(q, g2 <= qb_top) : 0.0);
+            const T s = static_cast<T>(v);
+            put(out, at, s);
+            if (decltype(track)::value && __builtin_amdgcn_ballot_w64(s != T(0)) != 0)
+                top_b = max(top_b, g2);
+        };
+        int sto2 = sto;  // row of the second half's group
+        // Above G0 (the first step's second half) the zero coefficients give
+        // zeros, stored at G0's row and overwritten by the next step.
+        auto step = [&](auto slot, int g, int buf, auto track) {
+            constexpr int k = decltype(slot)::value;
+            const RoleForm c = cn;
+            cn = read_form(k + 1 < R ? buf : buf ^ 1, (k + 1) % R);
+            const int at = ld;
+            fetch((k + D) % RING, at);
+            ld = max(at - row, 0);
+            // each step's loads stay in its own issue slots, so the ring keeps
+            // its depth (and its registers)
+            __builtin_amdgcn_sched_barrier(0);
+            const double v = one.template step<SRC, STRAG>(
+                c, rF[k % RING], rf[k % RING],
+                STRAG && g > 0 ? static_cast<double>(rF[(k + 1) % RING]) : 0.0,
+                SRC ? source(rQa[k % RING], g <= qa_top) : 0.0);
+            const T s = static_cast<T>(v);
+            if (DOSE) {
+                dose = fma(v, c.c[7], dose);
+                psum += v;
+            }
+            if (decltype(track)::value && __builtin_amdgcn_ballot_w64(s != T(0)) != 0)
+                top_a = max(top_a, g);
+            if (XOUT) put(xout, sto, s);
+            if (!PAIR) {
+                put(out, sto, s);
+            } else {
+                const T o = swap_pair(s);
+                const double Pn = role ? s : o, Rn = role ? o : s;
+                second(g + 1, sto2, Pn, rQb[(k + D) % RING], track);
+                fetch_qb((k + D) % RING, at);
+                P2 = Pn;
+                R2 = Rn;
+                c2 = c;
+            }
+            sto2 = sto;
+            sto -= row;
+        };
+        // at the top of a chunk (group g0 in slot 0): the next chunk's
+        // coefficients into the other buffer, those after it into registers
+        auto chunk = [&](int g0, int buf) {
+            stage_store(buf ^ 1);
+            stage_load(g0 - 2 * R);
+            wave_lds_sync();
+        };
+        using Yes = std::true_type;
+        int g0 = G0, buf = 0;
+        for (; g0 >= R - 1 && (top_a < 0 || (PAIR && top_b < 0)); g0 -= R, buf ^= 1) {
+            chunk(g0, buf);
+            unroll<R>([&](auto k) { step(k, g0 - decltype(k)::value, buf, Yes{}); });
+        }
+        for (; g0 >= R - 1; g0 -= R, buf ^= 1) {
+            chunk(g0, buf);
+            unroll<R>([&](auto k) { step(k, g0 - decltype(k)::value, buf, std::false_type{}); });
+        }
+        if (g0 >= 0) {
+            chunk(g0, buf);
+            unroll<R>([&](auto k) {  // tail: groups g0 .. 0 (fewer than R)
+                if (decltype(k)::value <= g0) step(k, g0 - decltype(k)::value, buf, Yes{});
+            });
+        }
+        if (PAIR)  // group 0 has no lower neighbour
+            second(0, 0, 0.0, SRC ? bload<T>(bb, voff, 0) : T(0), Yes{});
+    }
+    if (DOSE) {  // partials: dose (both roles), proxy (role 0)
+        double d = live ? dose * yzw[lane / nang] : 0.0, p = live && !role ? psum : 0.0;
+        for (int off = 32; off > 0; off >>= 1) {
+            d += __shfl_xor(d, off);
+            p += __shfl_xor(p, off);
+        }
+        if (threadIdx.x == 0) {
+            partials[blockIdx.x] = d;
+            if (proxy) partials[gridDim.x + blockIdx.x] = p;
+        }
+    }
+    if (threadIdx.x == 0) {
+        const int t = PAIR ? top_b : top_a;
+        if (tops.out && t >= 0) atomicMax(tops.out, t);
+        if (tops.out_x && top_a >= 0) atomicMax(tops.out_x, top_a);
+    }
+}
+
 // First-order implicit upwind energy step: the reference's legacy energy
 // model (energyDgCnKernel, use_legacy branch, src/energy_solver.cu:88-106)
 // and its lite-memory primary step (litePrimaryEnergyStepKernel,
@@ -552,7 +810,7 @@ template <typename T, int LPT, bool SRC, bool STRAG>
 void dispatch_pair(T* F, T* f, const EnergyCoef* coef, const T* Qa, const T* Qb, T* XF, T* Xf,
                    const unsigned* xmask, int Ng, long long lanes, const double* yzw, int nang,
                    double* partials, bool proxy, hipStream_t s, const SweepTops& tops) {
-    const int blocks = energy_blocks(lanes, sizeof(T));
+    const int blocks = energy_blocks(lanes, Ng, sizeof(T));
     BFPN_REQUIRE(lanes < (1LL << 31), "energy sweep indexes lanes with 32-bit offsets");
     if (XF)
         hipLaunchKernelGGL((energy_pair_kernel<T, LPT, SRC, STRAG, true>), dim3(blocks),
@@ -569,6 +827,18 @@ void dispatch_pair_lpt(T* F, T* f, const EnergyCoef* coef, const T* Qa, const T*
                        T* Xf, const unsigned* xmask, int Ng, long long lanes, const double* yzw,
                        int nang, double* partials, bool proxy, hipStream_t s,
                        const SweepTops& tops) {
+    if (energy_split(lanes, Ng, sizeof(T))) {
+        const dim3 grid(energy_blocks(lanes, Ng, sizeof(T)));
+        if (XF)
+            hipLaunchKernelGGL((energy_split_kernel<T, true, SRC, STRAG, true, true>), grid,
+                               dim3(64), 0, s, F, f, coef, Qa, Qb, XF, Xf, Ng,
+                               static_cast<int>(lanes), yzw, nang, partials, proxy ? 1 : 0, tops);
+        else
+            hipLaunchKernelGGL((energy_split_kernel<T, true, SRC, STRAG, true, false>), grid,
+                               dim3(64), 0, s, F, f, coef, Qa, Qb, XF, Xf, Ng,
+                               static_cast<int>(lanes), yzw, nang, partials, proxy ? 1 : 0, tops);
+        return;
+    }
     if constexpr (sizeof(T) == 4) {
         const int lpt = lanes_per_thread(lanes, sizeof(T));
         if (lpt == 4)
@@ -583,7 +853,7 @@ template <typename T, int LPT, bool SRC, bool STRAG>
 void dispatch_dose(T* F, T* f, const EnergyCoef* coef, const T* Q1, int Ng, long long lanes,
                    const double* yzw, int nang, double* partials, bool proxy, hipStream_t s,
                    const SweepTops& tops) {
-    const int blocks = energy_blocks(lanes, sizeof(T));
+    const int blocks = energy_blocks(lanes, Ng, sizeof(T));
     BFPN_REQUIRE(lanes < (1LL << 31), "energy sweep indexes lanes with 32-bit offsets");
     if (partials)
         hipLaunchKernelGGL((energy_half_kernel<T, LPT, SRC, STRAG, true>), dim3(blocks),
@@ -599,6 +869,19 @@ template <typename T, bool SRC, bool STRAG>
 void dispatch_lpt(T* F, T* f, const EnergyCoef* coef, const T* Q1, int Ng, long long lanes,
                   const double* yzw, int nang, double* partials, bool proxy, hipStream_t s,
                   const SweepTops& tops) {
+    if (energy_split(lanes, Ng, sizeof(T))) {
+        const dim3 grid(energy_blocks(lanes, Ng, sizeof(T)));
+        T* const none = nullptr;
+        if (partials)
+            hipLaunchKernelGGL((energy_split_kernel<T, false, SRC, STRAG, true, false>), grid,
+                               dim3(64), 0, s, F, f, coef, Q1, none, none, none, Ng,
+                               static_cast<int>(lanes), yzw, nang, partials, proxy ? 1 : 0, tops);
+        else
+            hipLaunchKernelGGL((energy_split_kernel<T, false, SRC, STRAG, false, false>), grid,
+                               dim3(64), 0, s, F, f, coef, Q1, none, none, none, Ng,
+                               static_cast<int>(lanes), yzw, nang, partials, 0, tops);
+        return;
+    }
     if constexpr (sizeof(T) == 4) {
         const int lpt = lanes_per_thread(lanes, sizeof(T));
         if (lpt == 4)
@@ -610,7 +893,8 @@ void dispatch_lpt(T* F, T* f, const EnergyCoef* coef, const T* Q1, int Ng, long 
 
 }  // namespace
 
-int energy_blocks(long long lanes, size_t elem) {
+int energy_blocks(long long lanes, int Ng, size_t elem) {
+    if (energy_split(lanes, Ng, elem)) return static_cast<int>((lanes + 31) / 32);
     const long long per_block = static_cast<long long>(kBlock) * lanes_per_thread(lanes, elem);
     return static_cast<int>((lanes + per_block - 1) / per_block);
 }

@@ -35,14 +35,14 @@ struct SweepTops {
 // null.  When dose != null each block writes FP64 partials:
 //   dose[block]        = sum w_yz(s) (F*w1[g] + f*w2[g])  over its lanes
 //   dose[nblk + block] = sum f                           (proxy), if proxy
-// The lanes handled by a block are [block*256, block*256+256).
 template <typename T>
 void launch_energy_half(T* F, T* f, const EnergyCoef* coef, const T* Q1, int Ng, long long lanes,
                         bool straggling, const double* yz_weight,
                         int nang, double* dose_partials, bool proxy, hipStream_t s,
                         const SweepTops& tops = SweepTops{});
-// Dose partials written by a sweep over `lanes` lanes of `elem`-byte state.
-int energy_blocks(long long lanes, size_t elem);
+// Dose partials written by a sweep over Ng groups of `lanes` lanes of
+// `elem`-byte state.
+int energy_blocks(long long lanes, int Ng, size_t elem);
 
 // Two consecutive energy half steps in one sweep (end of depth step n with
 // source Qa and the dose/proxy partials of step n, start of step n+1 with

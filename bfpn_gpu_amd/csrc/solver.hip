@@ -404,7 +404,7 @@ public:
         }
         for (int k = 0; k < 4; ++k) cur_[k] = state_[k].as<T>();
         eb_ = (P_->legacy || P_->lite) ? upwind_blocks(P_->lanes)
-                                       : energy_blocks(P_->lanes, sizeof(T));
+                                       : energy_blocks(P_->lanes, g.Ng, sizeof(T));
         partial_p_.ensure(4 * 2 * eb_ * sizeof(double));  // four slots: steps rotate
         partial_s_.ensure(eb_ * sizeof(double));
         grow_history(std::max(16, g.Nx));
@@ -512,7 +512,7 @@ public:
             for (size_t k = 0; k < sl.mat.size(); ++k) {
                 const bool maj = static_cast<int>(k) == sl.major;
                 const long long nodes_k = maj ? nyz : sl.count[k];
-                const int eb = energy_blocks(nodes_k * nang, sizeof(T));
+                const int eb = energy_blocks(nodes_k * nang, Ng, sizeof(T));
                 sl.eb.push_back(eb);
                 sl.poff.push_back(poff);
                 poff += 2 * eb;

@@ -1,0 +1,64 @@
+"""Grids of few lanes: the energy sweeps that share a lane between two threads.
+
+At the edges of that kernel (one lane, a ragged last wave, fewer groups than
+its ring and its coefficient chunks) against the sweeps of wide grids and the
+oracle.
+"""
+import numpy as np
+import pytest
+
+from gpu_cases import small_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("straggling,with_source", [(False, False), (True, False), (False, True),
+                                                     (True, True)])
+@pytest.mark.parametrize("lanes,Ng", [(1, 1), (31, 2), (32, 15), (33, 16), (97, 17), (64, 31),
+                                      (130, 32), (63, 50)])
+def test_half_sweep_equals_the_wide_grid_sweep(gpu, dtype, straggling, with_source, lanes, Ng):
+    """The same lanes alone and as the first columns of a grid of 2^16 lanes
+    and more (one thread per lane): the same operations on every value, so the
+    same bits."""
+    rng = np.random.default_rng(100 * lanes + Ng)
+    wide = (1 << 16) + 32
+    h, dg, rho = 0.01, 0.518, 1.1
+    S = 5.0 + 100.0 * rng.random(Ng + 1)
+    sig, T = 0.02 * rng.random(Ng), 0.01 * rng.random(Ng)
+    F = rng.standard_normal((Ng, wide)).astype(dtype)
+    f = (0.3 * rng.standard_normal((Ng, wide))).astype(dtype)
+    Q = rng.random((Ng, wide)).astype(dtype) if with_source else None
+    tabs = [gpu.DeviceArray(a) for a in (S, sig, T)]
+
+    def run(cols):
+        a, b = (gpu.DeviceArray(np.ascontiguousarray(x[:, :cols])) for x in (F, f))
+        q = gpu.DeviceArray(np.ascontiguousarray(Q[:, :cols])) if with_source else None
+        gpu.ops.energy_half(a, b, *tabs, h, dg, rho, Ng, cols, 1, Q1=q, straggling=straggling)
+        return a.numpy()[:, :lanes], b.numpy()[:, :lanes]
+
+    for narrow, full in zip(run(lanes), run(wide)):
+        np.testing.assert_array_equal(narrow, full)
+
+
+@pytest.mark.parametrize("Ng,over", [(17, dict(Ny=2, Nz=1, Nmu=2, Nom=3)),
+                                     (33, dict(Ny=3, Nz=2, Nmu=3, Nom=3)),
+                                     (500, dict(Ny=6, Nz=5, Nmu=5, Nom=5))])
+@pytest.mark.parametrize("straggling", [0, 1])
+def test_paired_sweeps_at_group_and_lane_edges(gpu, oracle_mod, Ng, over, straggling):
+    """Whole steps with the secondary (paired sweeps with two sources) against
+    the oracle, and in one call against one call per step, bit for bit."""
+    c = small_case(Ng=Ng, Lg=259.0 * Ng / 500, energy=1.0 + 0.4 * 259.0 * Ng / 500,
+                   flags=dict(eq15_straggling=straggling), **over)
+    ref = oracle_mod.Solver(c)
+    ref.advance(5)
+    for precision, tol in ((gpu.FP64, 1e-10), (gpu.FP32, 2e-4)):
+        with gpu.Solver(c, precision) as one, gpu.Solver(c, precision) as many:
+            one.advance(5)
+            for _ in range(5):
+                many.advance(1)
+            np.testing.assert_array_equal(one.history()[0], many.history()[0])
+            for k in range(4):
+                a, r = one.state(k), ref.state(k)
+                np.testing.assert_array_equal(a, many.state(k))
+                assert np.abs(a - r).max() <= tol * max(np.abs(r).max(), 1e-300)
