@@ -228,9 +228,12 @@ void launch_energy_moments(const T* F, const T* f, const T* F1, const T* f1, int
                            double weight, double* partials, double* out, hipStream_t s);
 
 // Y-Z dose plane (nyz doubles): per node, the Eq.24 dose weights of `coef`
-// applied to psi^1 and psi^2, summed over groups and directions, times scale.
+// applied to psi^1 and psi^2, summed over groups and directions, times scale;
+// partials: spot_partial_count doubles.
+size_t spot_partial_count(int Ng, int nyz);
 template <typename T>
 void launch_spot_plane(const T* F, const T* f, const T* F1, const T* f1, const EnergyCoef* coef,
-                       int Ng, int nyz, int nang, double scale, double* plane, hipStream_t s);
+                       int Ng, int nyz, int nang, double scale, double* partials, double* plane,
+                       hipStream_t s);
 
 }  // namespace bfpn

@@ -572,10 +572,11 @@ public:
                                             "(not kept with --lite-memory)");
         sync_all();
         const int nyz = static_cast<int>(P_->nyz);
+        diag_part_.ensure(spot_partial_count(grid.Ng, nyz) * sizeof(double));
         diag_out_.ensure(static_cast<size_t>(nyz) * sizeof(double));
         launch_spot_plane<T>(cur_[0], cur_[1], cur_[2], cur_[3], P_->coef.template as<EnergyCoef>(),
                              grid.Ng, nyz, P_->nang, d.du * d.dv / P_->density,
-                             diag_out_.as<double>(), stream);
+                             diag_part_.as<double>(), diag_out_.as<double>(), stream);
         BFPN_HIP(hipStreamSynchronize(stream));
         BFPN_HIP(hipMemcpy(host, diag_out_.as<double>(), static_cast<size_t>(nyz) * sizeof(double),
                            hipMemcpyDeviceToHost));
