@@ -39,7 +39,8 @@ def test_dose_over_chunks(gpu, oracle_mod, dtype, have, Ng, Ny, Nz, nang):
                                      (17, dict(Ny=2, Nz=3, Nmu=7, Nom=9)),
                                      (65, dict(Ny=4, Nz=2, Nmu=8, Nom=9))])
 def test_dose_plane_over_chunks(gpu, oracle_mod, Ng, over):
-    c = small_case(Ng=Ng, Lg=259.0 * Ng / 500, **over)
+    c = small_case(Ng=Ng, Lg=259.0 * Ng / 500, energy=1.0 + 0.2 * Ng,
+                   flags=dict(normalize_initial_mass=0, discrete_angle_delta=0), **over)
     d = oracle_mod.deltas(c)
     rng = np.random.default_rng(Ng)
     st = [rng.random(c.cells) for _ in range(4)]
