@@ -46,7 +46,11 @@ namespace {
 //     X'^T = Su^T W^T        (A = Su chained,   B = W)
 // using the symmetry of the DST-I bases; X'^T leaves the last stage with 4
 // consecutive elements of a plane row per lane and is stored straight back.
-// V4: Nom % 4 == 0 -- rows are read and written as 16-byte vectors.
+// V4 (Nom >= 4): rows are read and written as 16-byte vectors, columns 4k .. of
+// a row per vector.  Where Nom is no multiple of 4 the row's last vector holds
+// its last four columns instead and overlaps the one before: the plan stores
+// the bases' columns (stage 1, the repeated ones as zeros) and rows (stage 4,
+// where both lanes compute the same value) in that order, angle_column().
 template <int MT, int NT, bool V4>
 __global__ __launch_bounds__(256) void angle_mfma_kernel(float* __restrict__ F,
                                                          const float* __restrict__ factors,
@@ -94,14 +98,20 @@ __global__ __launch_bounds__(256) void angle_mfma_kernel(float* __restrict__ F,
 #pragma unroll
         for (int h = 0; h < 2; ++h)
             ld_off[mt][h] = static_cast<unsigned>(
-                (min(mt * 16 + i, Nmu - 1) * Nom + min(8 * q + 4 * h, max(Nom - 4, 0))) * sizeof(float));
+                (min(mt * 16 + i, Nmu - 1) * Nom +
+                 (V4 ? min(8 * q + 4 * h, max(Nom - 4, 0)) : min(8 * q, Nom - 1))) * sizeof(float));
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             const int v = mt * 16 + i, a0 = nt * 16 + 4 * q;
-            st_off[mt][nt] = (v < Nmu && a0 < Nom) ? static_cast<unsigned>((v * Nom + a0) * sizeof(float))
-                                                   : kOutside;
+            const int first = V4 ? min(a0, Nom - 4) : a0;
+            st_off[mt][nt] = (v < Nmu && a0 < Nom)
+                                 ? static_cast<unsigned>((v * Nom + first) * sizeof(float))
+                                 : kOutside;
         }
     }
+    // Rows of fewer than 4 columns: a lane's columns are clamped to the row's
+    // last, and its 4-column output groups are cut there.
+    const int e_max = max(Nom - 1 - 8 * q, 0);
     // Fragment of constant `a` (0 Su, 1 Su chained, 2 Sv chained), tile t,
     // at compile-time offsets from the lane's base (row i, columns 8q..).
     auto frag = [&](const _Float16* base, int a, int t) {
@@ -120,7 +130,6 @@ __global__ __launch_bounds__(256) void angle_mfma_kernel(float* __restrict__ F,
         int oz;
         asm volatile("v_mov_b32 %0, 0" : "=v"(oz));
         const _Float16* cb = &cst[0][i][8 * q] + oz;
-        float* X = F + static_cast<long long>(p) * na;
         const unsigned so = static_cast<unsigned>((p - p0) * na * static_cast<int>(sizeof(float)));
         if (g != g_cur) {  // CN factors of this group, in the D layout, / 256
             g_cur = g;
@@ -143,7 +152,6 @@ __global__ __launch_bounds__(256) void angle_mfma_kernel(float* __restrict__ F,
         float x[MT][8];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            const float* row = X + min(mt * 16 + i, Nmu - 1) * Nom;
             if (V4) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
@@ -155,7 +163,8 @@ __global__ __launch_bounds__(256) void angle_mfma_kernel(float* __restrict__ F,
                 }
             } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) x[mt][e] = row[min(8 * q + e, Nom - 1)];
+                for (int e = 0; e < 8; ++e)
+                    x[mt][e] = bload<float>(Fw, ld_off[mt][0] + 4u * min(e, e_max), so);
             }
         }
         // the plane's scale s = 2^(4 - floor(log2 max|X|)) (biased exponent
@@ -220,7 +229,6 @@ __global__ __launch_bounds__(256) void angle_mfma_kernel(float* __restrict__ F,
                 w[4 + r] = NT > 1 ? d3[NT - 1][mt][r] : 0.f;
             }
             const HalfFrag2 b = split8_h<false>(w, one);
-            const int v = mt * 16 + i;
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 f32x4 d = mma_cs(frag(cb, 1, nt), b, zero4());
@@ -232,8 +240,157 @@ __global__ __launch_bounds__(256) void angle_mfma_kernel(float* __restrict__ F,
                 } else {
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
-                        if (v < Nmu && a0 + r < Nom) X[v * Nom + a0 + r] = d[r];
+                        bstore(d[r], Fw, a0 + r < Nom ? st_off[mt][nt] + 4u * r : kOutside, so);
                 }
+            }
+        }
+    }
+}
+
+// Planes of at most 16 x 16 directions: one 16 x 16 tile per stage, the same
+// split FP16 arithmetic and stage chaining as above (a stage's D tile is the
+// next one's operand as it is), with the constant fragments in registers and
+// no LDS; results are those of the kernel above bit for bit (mfma.hpp).
+// Planes of at most 8 rows (PM2) or columns (PN2) share a tile, two along that
+// axis at stride 8, with block-diagonal bases: up to four planes for the issue
+// of one; each keeps its own scale, and a tile with a value that is not finite
+// runs plane by plane, so that it spoils its own plane only.  A lane holds 4
+// columns 4q .. of row i, read through a buffer resource at fixed offsets
+// (outside the plane: past the resource, which reads 0 and drops stores), one
+// tile ahead of the arithmetic.  VEC: Nom >= 4, one 16-byte vector per lane,
+// the row's last one overlapping as above.
+// What bounds it: HBM and issue about equally (80 vector operations and 2
+// accesses per tile).  The general kernel padded these planes to K = 32, read
+// 8 clamped values per lane and stored under branches.  Measured, per call with
+// the general kernel and with this one: 13 x 13 directions (29.8 M cells, HBM
+// floor 42 us) 104 -> 44 us, 11 x 11 (26.7 M) 114 -> 47, 10 x 10 (12.8 M)
+// 61 -> 33, 7 x 7 (2 M, launch included) 23 -> 13.
+template <bool PM2, bool PN2, bool VEC>
+__global__ __launch_bounds__(256) void angle_small_kernel(float* __restrict__ F,
+                                                          const float* __restrict__ factors,
+                                                          AnglePlan plan, int planes, int per_wave,
+                                                          int nyz, int Nmu, int Nom, float one,
+                                                          const int* __restrict__ top) {
+    constexpr int NPN = PN2 ? 2 : 1, P = (PM2 ? 2 : 1) * NPN;  // planes per tile
+    const int Ng = planes / nyz;
+    const int active = top ? min(planes, (min(*top, Ng - 1) + 1) * nyz) : planes;
+    const int waves = gridDim.x * 4;
+    const int pw = top ? ((active + waves - 1) / waves + P - 1) / P * P : per_wave;
+    const int lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
+    int p = __builtin_amdgcn_readfirstlane((blockIdx.x * 4 + (threadIdx.x >> 6)) * pw);
+    const int p_end = min(active, p + pw);
+    if (p >= p_end) return;
+    const int na = Nmu * Nom;
+    const int p0 = p;
+    const __amdgpu_buffer_rsrc_t Fw =
+        make_rsrc(F + static_cast<long long>(p0) * na,
+                  static_cast<unsigned>(static_cast<long long>(p_end - p0) * na * sizeof(float)));
+    // Coordinates of a tile index x (0 .. 15) along an axis packed or not:
+    // block and index inside it.
+    auto blk = [](bool two, int x) { return two ? x >> 3 : 0; };
+    auto idx = [](bool two, int x) { return two ? x & 7 : x; };
+    // load / store layout: row i, columns 4q ..; the lane's plane in the tile
+    const int v = idx(PM2, i), a0 = idx(PN2, 4 * q), lp = blk(PM2, i) * NPN + blk(PN2, 4 * q);
+    unsigned off[VEC ? 1 : 4];
+#pragma unroll
+    for (int r = 0; r < (VEC ? 1 : 4); ++r) {
+        const int c = VEC ? min(a0, Nom - 4) : a0 + r;
+        off[r] = v < Nmu && a0 + r < Nom
+                     ? static_cast<unsigned>((lp * na + v * Nom + c) * sizeof(float))
+                     : kOutside;
+    }
+    // constant fragments: element (i, 4q + r) of the block-diagonal bases, Su's
+    // columns (stage 1) and rows (stage 4) in vector order (Su for stage 4 and
+    // Sv are stored with their columns chained: index 4k + r in slot 8k + r)
+    auto constant = [](const _Float16* h, const _Float16* l, int at, bool diagonal) {
+        Const16 f;
+        f.hi = *reinterpret_cast<const f16x4*>(h + at);
+        f.lo = *reinterpret_cast<const f16x4*>(l + at);
+        if (!diagonal) f.hi = f.lo = f16x4{};
+        return f;
+    };
+    auto wide = [](const Const16& f) {
+        const f16x4 z{};
+        return Const32{__builtin_shufflevector(f.lo, z, 0, 1, 2, 3, 4, 5, 6, 7),
+                       __builtin_shufflevector(z, f.hi, 0, 1, 2, 3, 4, 5, 6, 7),
+                       __builtin_shufflevector(f.hi, z, 0, 1, 2, 3, 4, 5, 6, 7)};
+    };
+    const bool du = blk(PN2, i) == blk(PN2, 4 * q), dv = blk(PM2, i) == blk(PM2, 4 * q);
+    const Const16 su = constant(plan.su_h, plan.su_l, idx(PN2, i) * 32 + idx(PN2, 4 * q), du);
+    const Const32 sup =
+        wide(constant(plan.sup_h, plan.sup_l, idx(PN2, i) * 32 + 2 * idx(PN2, 4 * q), du));
+    const Const32 sv =
+        wide(constant(plan.svp_h, plan.svp_l, idx(PM2, i) * 32 + 2 * idx(PM2, 4 * q), dv));
+    // CN factors in the layout of stage 2's result: nu = 4q + r, mu = i
+    const int nu0 = idx(PM2, 4 * q), mu = idx(PN2, i), lpd = blk(PM2, 4 * q) * NPN + blk(PN2, i);
+    f32x4 cf = zero4();
+    int g_cur = -1;
+    int g = p / nyz, s_in = p - g * nyz;  // group and node of the tile's first plane (uniform)
+
+    auto load = [&](int at) {
+        const unsigned so = static_cast<unsigned>((at - p0) * na * static_cast<int>(sizeof(float)));
+        const bool mine = P == 1 || at + lp < p_end;  // (a run's last tile may be part full)
+        f32x4 x;
+        if constexpr (VEC) {
+            const float4 t = bload4(Fw, mine ? off[0] : kOutside, so);
+            x = f32x4{t.x, t.y, t.z, t.w};
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[r] = bload<float>(Fw, mine ? off[r] : kOutside, so);
+        }
+        return x;
+    };
+    f32x4 next = load(p);
+    for (; p < p_end; p += P) {
+        const f32x4 x = next;
+        next = load(p + P < p_end ? p + P : p);
+        const bool straddles = P > 1 && s_in + P > nyz;  // planes of more than one group
+        if (g != g_cur || straddles) {
+            constexpr float kUnscale = 1.0f / (kAngleBasisScale * kAngleBasisScale);
+            const int gl = straddles ? min(g + (s_in + lpd) / nyz, Ng - 1) : g;
+            const float* C = factors + static_cast<long long>(gl) * na;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                cf[r] = nu0 + r < Nmu && mu < Nom ? C[(nu0 + r) * Nom + mu] * kUnscale : 0.f;
+            g_cur = straddles ? -1 : g;
+        }
+        for (s_in += P; s_in >= nyz; s_in -= nyz) ++g;
+        const unsigned so = static_cast<unsigned>((p - p0) * na * static_cast<int>(sizeof(float)));
+        // the planes of `x` (a lane of another plane: zeros, and not `mine`)
+        auto sandwich = [&](f32x4 x, float mx, bool mine) {
+            // each plane's scale, as in angle_mfma_kernel
+            const int sb = min(max(258 - (__float_as_int(mx) >> 23), 1), 253);
+            const float sc = __int_as_float(sb << 23);
+            const float unscale =
+                __int_as_float((254 - sb) << 23) / (kAngleBasisScale * kAngleBasisScale);
+            f16x4 xh, xl;
+            split4_h<true>(x, sc, xh, xl);
+            const f32x4 y = mma16_sc(xh, xl, su);                    // Y  = X Su^T
+            const f32x4 z = mma32_cs(sv, split44_h(y, one)) * cf;    // Z  = C (.) (Sv Y)
+            const f32x4 w = mma32_sc(split44_h(z, one), sv);         // W^T = Z^T Sv
+            const f32x4 d = mma32_cs(sup, split44_h(w, one)) * unscale;  // X'^T = Su^T W^T
+            if constexpr (VEC) {
+                bstore4(make_float4(d[0], d[1], d[2], d[3]), Fw, mine ? off[0] : kOutside, so);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) bstore(d[r], Fw, mine ? off[r] : kOutside, so);
+            }
+        };
+        if constexpr (P == 1) {
+            float mx = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+            sandwich(x, wave_max_nonneg(mx), true);
+        } else {
+            unsigned u = 0;  // the plane's largest |value| as bits (above infinity's: NaN)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) u = max(u, __float_as_uint(x[r]) & 0x7fffffffu);
+            u = block_max_bits<PM2, PN2>(u);
+            const bool mine = p + lp < p_end;
+            if (__builtin_amdgcn_ballot_w64(u >= 0x7f800000u) == 0) {
+                sandwich(x, __uint_as_float(u), mine);
+            } else {
+                for (int k = 0; k < P; ++k)
+                    sandwich(lp == k ? x : zero4(), __uint_as_float(min(u, 0x7f800000u)),
+                             mine && lp == k);
             }
         }
     }
@@ -320,24 +477,40 @@ void launch_angle_mfma(float* F, const float* factors, const AnglePlan& plan, in
     if (planes == 0) return;
     BFPN_REQUIRE(planes * Nmu * Nom < (1LL << 31) && planes < (1LL << 30),
                  "MFMA DST indexes planes with 32-bit offsets");
-    // 8192 waves (32 per CU) walking contiguous runs of planes
-    const int waves = static_cast<int>(std::min<long long>(planes, 8192));
-    const int per_wave = static_cast<int>((planes + waves - 1) / waves);
-    const int blocks = (static_cast<int>((planes + per_wave - 1) / per_wave) + 3) / 4;
-    const dim3 grid(blocks), block(256);
-    const int mt = Nmu > 16 ? 2 : 1, nt = Nom > 16 ? 2 : 1;
-#define BFPN_ANGLE(MT_, NT_, V4_)                                                              \
-    hipLaunchKernelGGL((angle_mfma_kernel<MT_, NT_, V4_>), grid, block, 0, s, F, factors, plan,\
-                       static_cast<int>(planes), per_wave, nyz, Nmu, Nom, 1.0f, top)
-#define BFPN_ANGLE_V(MT_, NT_)                                                                 \
-    if (Nom % 4 == 0) BFPN_ANGLE(MT_, NT_, true);                                              \
-    else BFPN_ANGLE(MT_, NT_, false)
-    if (mt == 2 && nt == 2) { BFPN_ANGLE_V(2, 2); }
-    else if (mt == 2) { BFPN_ANGLE_V(2, 1); }
-    else if (nt == 2) { BFPN_ANGLE_V(1, 2); }
-    else { BFPN_ANGLE_V(1, 1); }
-#undef BFPN_ANGLE_V
-#undef BFPN_ANGLE
+    // 8192 waves (32 per CU) walking contiguous runs of planes, in tiles of
+    // planes_per_tile
+    auto shape = [&](int planes_per_tile, int& per_wave) {
+        const long long tiles = (planes + planes_per_tile - 1) / planes_per_tile;
+        const long long waves = std::min<long long>(tiles, 8192);
+        per_wave = static_cast<int>((tiles + waves - 1) / waves) * planes_per_tile;
+        return (static_cast<int>((planes + per_wave - 1) / per_wave) + 3) / 4;
+    };
+    int per_wave = 0;
+    auto go = [&](auto kernel, int planes_per_tile) {
+        const int blocks = shape(planes_per_tile, per_wave);
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, s, F, factors, plan,
+                           static_cast<int>(planes), per_wave, nyz, Nmu, Nom, 1.0f, top);
+    };
+    const bool vec = Nom >= 4;
+    if (Nmu <= 16 && Nom <= 16) {
+        if (Nmu <= 8 && Nom <= 8) {
+            if (vec) go(&angle_small_kernel<true, true, true>, 4);
+            else go(&angle_small_kernel<true, true, false>, 4);
+        } else if (Nmu <= 8) {
+            go(&angle_small_kernel<true, false, true>, 2);
+        } else if (Nom <= 8) {
+            if (vec) go(&angle_small_kernel<false, true, true>, 2);
+            else go(&angle_small_kernel<false, true, false>, 2);
+        } else {
+            go(&angle_small_kernel<false, false, true>, 1);
+        }
+    } else if (Nom > 16) {
+        if (Nmu > 16) go(&angle_mfma_kernel<2, 2, true>, 1);
+        else go(&angle_mfma_kernel<1, 2, true>, 1);
+    } else {
+        if (vec) go(&angle_mfma_kernel<2, 1, true>, 1);
+        else go(&angle_mfma_kernel<2, 1, false>, 1);
+    }
     BFPN_HIP(hipGetLastError());
 }
 

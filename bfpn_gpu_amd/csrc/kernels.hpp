@@ -157,8 +157,10 @@ void launch_angle_full(T* F, const T* factors, const T* su, const T* sv, int Ng,
 
 // Sine bases of the MFMA DST: 16 x the basis (a power of two, exact), split
 // into two FP16 terms (hi + lo) from the FP64 values, 32x32 zero padded,
-// row-major: Su as is, and Su and Sv with their columns in the
-// register-chaining order of the DST kernel.
+// row-major: Su with its columns in the order of a row's vectors
+// (angle_column, repeated columns zero), Su with its rows in that order and
+// its columns in the register-chaining order of the DST kernel, and Sv with
+// its columns chained.
 constexpr float kAngleBasisScale = 16.0f;
 struct AnglePlan {
     const _Float16* su_h = nullptr;
@@ -168,6 +170,14 @@ struct AnglePlan {
     const _Float16* svp_h = nullptr;
     const _Float16* svp_l = nullptr;
 };
+// Column of a plane row of n values that slot k of its 4-value vectors holds:
+// the row's last vector holds its last four columns (-1: no such vector).
+// Slots whose column is below the vector's first, angle_column(k) < (k & ~3),
+// repeat one of the vector before.
+constexpr int angle_column(int k, int n) {
+    const int first = k & ~3;
+    return first >= n || (n < 4 && k >= n) ? -1 : (n < 4 || first + 3 < n) ? k : n - 4 + (k & 3);
+}
 // K slot 8q + 4u + r of a chained MFMA operand <-> matrix index 16u + 4q + r.
 constexpr int chain_index(int slot) { return 16 * ((slot & 7) >> 2) + 4 * (slot >> 3) + (slot & 3); }
 // FP32 DST on the matrix cores (Nmu, Nom <= 32), in place.

@@ -121,6 +121,69 @@ __device__ inline f32x4 mma_cs(const HalfFrag2& a, const HalfFrag2& b, f32x4 acc
     return acc;
 }
 
+// Planes of at most 16 x 16: lane holds 4 values 4q .. 4q+3 of row lane%16, the
+// operand layout of v_mfma_f32_16x16x16_f16 and the D layout of every product.
+typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
+template <bool SCALE>
+__device__ inline void split4_h(f32x4 x, float s, f16x4& hi, f16x4& lo) {
+    hi = __builtin_convertvector(SCALE ? x * s : x, f16x4);
+    const f32x4 h = __builtin_convertvector(hi, f32x4);
+    f32x4 r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = __builtin_fmaf(x[e], s, -h[e]);
+    lo = __builtin_convertvector(r, f16x4);
+}
+// The three products of mma_sc / mma_cs in their order.  The hardware rounds
+// after each group of 8 K slots held by one lane (x32) or by two (x16), and
+// sums inside a group do not depend on the slots' order (measured); so the x16
+// form equals the x32 form over the natural K order, and for the chained order,
+// 4 values per lane, one x32 operand holds both terms of the state, {hi, lo},
+// against constants whose other half is zero.
+struct Const16 {
+    f16x4 hi, lo;
+};
+struct Const32 {
+    f16x8 lo_0, zero_hi, hi_0;  // {c_lo, 0}, {0, c_hi}, {c_hi, 0}
+};
+__device__ inline f32x4 mma16_sc(f16x4 hi, f16x4 lo, const Const16& c) {
+    f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x16f16(hi, c.lo, zero4(), 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x16f16(lo, c.hi, acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(hi, c.hi, acc, 0, 0, 0);
+}
+__device__ inline f32x4 mma32_sc(f16x8 x, const Const32& c) {
+    f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, c.lo_0, zero4(), 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, c.zero_hi, acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(x, c.hi_0, acc, 0, 0, 0);
+}
+__device__ inline f32x4 mma32_cs(const Const32& c, f16x8 x) {
+    f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(c.lo_0, x, zero4(), 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(c.zero_hi, x, acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(c.hi_0, x, acc, 0, 0, 0);
+}
+__device__ inline f16x8 split44_h(f32x4 x, float one) {
+    f16x4 hi, lo;
+    split4_h<false>(x, one, hi, lo);
+    return __builtin_shufflevector(hi, lo, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// Maximum of u over a block of lanes, in every lane of it: rows of 16 lanes
+// (HALF: 8), all four rows of the wave (PAIRS: rows 0-1 and 2-3 apart).
+template <bool HALF, bool PAIRS>
+__device__ inline unsigned block_max_bits(unsigned u) {
+    u = max(u, static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(u), 0xB1, 0xF, 0xF, false)));
+    u = max(u, static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(u), 0x4E, 0xF, 0xF, false)));
+    u = max(u, static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(u), 0x141, 0xF, 0xF, false)));
+    if (!HALF)
+        u = max(u, static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(u), 0x140, 0xF, 0xF, false)));
+    const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);  // rows 0, 1 and 2, 3
+    u = max(a[0], a[1]);
+    if (!PAIRS) {
+        const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);  // halves of the wave
+        u = max(b[0], b[1]);
+    }
+    return u;
+}
+
 // Maximum of non-negative v over the wave, as a wave-uniform value: DPP
 // maxima within each row of 16 lanes (neighbour pairs, quads, half-row and
 // row mirrors), then the four rows' results read into scalar registers.  On

@@ -190,17 +190,19 @@ double half_value(uint16_t b) {
 }  // namespace
 
 void AnglePlanBuffers::build(int Nmu, int Nom, hipStream_t) {
-    // Su, Su (chained columns), Sv (chained columns); each zero padded to
-    // 32x32, scaled by kAngleBasisScale (exact) and split into FP16 hi + lo
-    // from the FP64 basis.  (The scale keeps the smallest basis values' lo
+    // Su (columns in vector order), Su (rows in vector order, columns
+    // chained), Sv (columns chained); each zero padded to 32x32, scaled by
+    // kAngleBasisScale (exact) and split into FP16 hi + lo from the FP64
+    // basis.  (The scale keeps the smallest basis values' lo
     // terms clear of the FP16 subnormal range.)
     std::vector<double> pad(3 * 32 * 32, 0.0);
     const auto su = sine_basis(Nom), sv = sine_basis(Nmu);
     for (int r = 0; r < 32; ++r)
         for (int c = 0; c < 32; ++c) {
             const int cc = chain_index(c);
-            if (r < Nom && c < Nom) pad[r * 32 + c] = su[r * Nom + c];
-            if (r < Nom && cc < Nom) pad[1024 + r * 32 + c] = su[r * Nom + cc];
+            const int vr = angle_column(r, Nom), vc = angle_column(c, Nom);
+            if (r < Nom && vc >= (c & ~3)) pad[r * 32 + c] = su[r * Nom + vc];
+            if (vr >= 0 && cc < Nom) pad[1024 + r * 32 + c] = su[vr * Nom + cc];
             if (r < Nmu && cc < Nmu) pad[2048 + r * 32 + c] = sv[r * Nmu + cc];
         }
     std::vector<uint16_t> vh(pad.size()), vl(pad.size());

@@ -1,0 +1,58 @@
+"""The DST over direction planes of every packing: planes that share a tile,
+ragged rows, planes of one and two tiles, tiles that hold planes of two energy
+groups or end a run part full.
+
+Each plane is checked against its own maximum, over magnitudes from 1e-25 to
+1e20: planes that share a tile keep their own scale.  Tolerance: the products
+carry about 2^-22 (three FP16 products) and sums are FP32; on random 20 x 20
+planes that makes 2.3e-7 of the maximum, and 1e-5 leaves the factor 40 by
+which single planes of a few values may exceed it.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("Nmu,Nom", [(1, 1), (2, 3), (4, 4), (5, 8), (8, 5), (8, 8), (7, 7), (8, 9),
+                                     (9, 8), (3, 16), (16, 2), (11, 11), (12, 12), (16, 16),
+                                     (9, 13), (17, 3), (17, 6), (20, 17), (5, 19), (16, 18),
+                                     (32, 31)])
+@pytest.mark.parametrize("nyz,Ng", [(1, 7), (3, 5), (6, 4), (25, 2)])
+def test_planes_against_the_oracle(gpu, oracle_mod, Nmu, Nom, nyz, Ng):
+    rng = np.random.default_rng(1000 * Nmu + 10 * Nom + nyz)
+    scale = 10.0 ** rng.uniform(-25, 20, (Ng, nyz, 1, 1))
+    F = (rng.standard_normal((Ng, nyz, Nmu, Nom)) * scale).astype(np.float32)
+    F[0, 0] = 0.0  # an empty plane stays empty beside others
+    sig = rng.uniform(0.0, 4.0, Ng)
+    args = (nyz, Ng, Nmu, Nom, 0.2, 0.13, 0.05, 1.2)
+    want = F.astype(np.float64).ravel()
+    oracle_mod.angle_full(want, sig, *args)
+    want = want.reshape(F.shape)
+    d = gpu.DeviceArray(F)
+    gpu.ops.angle_full(d, sig, *args)
+    got = d.numpy().reshape(F.shape).astype(np.float64)
+    top = np.abs(F).max(axis=(2, 3), keepdims=True).astype(np.float64)
+    assert np.all(np.abs(got - want) <= 1e-5 * top)
+    assert np.all(got[0, 0] == 0.0)
+
+
+@pytest.mark.parametrize("Nmu,Nom", [(7, 7), (4, 12), (12, 5), (11, 11), (20, 20)])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_a_plane_that_is_not_finite_spoils_itself_only(gpu, Nmu, Nom, bad):
+    nyz, Ng = 5, 4
+    rng = np.random.default_rng(3)
+    F = rng.standard_normal((Ng, nyz, Nmu, Nom)).astype(np.float32)
+    sig = rng.uniform(0.0, 4.0, Ng)
+    out = []
+    for spoil in (False, True):
+        G = F.copy()
+        if spoil:
+            G[1, 2, 0, 0] = G[3, 0, Nmu - 1, Nom - 1] = bad
+        d = gpu.DeviceArray(G)
+        gpu.ops.angle_full(d, sig, nyz, Ng, Nmu, Nom, 0.2, 0.13, 0.05, 1.2)
+        out.append(d.numpy().reshape(F.shape))
+    spoiled = np.zeros((Ng, nyz), bool)
+    spoiled[1, 2] = spoiled[3, 0] = True
+    np.testing.assert_array_equal(out[1][~spoiled], out[0][~spoiled])
+    assert np.all(np.isnan(out[1][spoiled]))
