@@ -10,12 +10,15 @@
 //     Y = Psi Su^T,  Z = coeff_g (.) (Sv Y),  W = Sv^T Z,  Psi' = W Su
 // runs per (g, s) plane of Nmu x Nom values, in place.  The CN factors
 // (ratio * DST normalisation) are built once on the host per (g, direction).
-// FP32 state: matrix cores, stages chained in registers (below).  FP64 state
-// or planes wider than 32: vector kernel with the plane and bases in LDS.
+// FP32 state: matrix cores, stages chained in registers (below).  FP64 state:
+// vector kernel, a thread per row or column of a plane.  Planes wider than 32:
+// vector kernel with the plane and bases in LDS.
 
 #include "buffer.hpp"
 #include "kernels.hpp"
 #include "mfma.hpp"
+
+#include <type_traits>
 
 namespace bfpn {
 namespace {
@@ -396,7 +399,136 @@ __global__ __launch_bounds__(256) void angle_small_kernel(float* __restrict__ F,
     }
 }
 
-// --------------------------------------------------- vector (FP64, wide) ---
+// ------------------------------------------------------- FP64, vector ------
+// FP64 planes of at most 32 x 32: one thread per row, then per column, then per
+// row of a plane, its line in registers, the bases through the scalar cache
+// (they are uniform, so a multiply-add reads its basis value from an SGPR and
+// needs one operand of the line).  The column pass does both inner stages and
+// the CN factors.  Planes pass through LDS between
+// the passes (rows padded to an odd pitch); HBM accesses are coalesced copies
+// of a work-group's run of planes.  Sizes are padded to those of dst_pitch(),
+// the bases with zeros.
+// The vector ALUs have the matrix cores' FP64 rate on this GPU, and 20 x 20
+// planes would pad to 32 x 32 tiles there (2.6 times the work).  Bound: HBM and
+// vector FP64 issue about equally (64 multiply-adds and 16 bytes per value at
+// 20 x 20).  The kernel below, one thread per value with both operands from
+// LDS: 1691 us for 21 x 21 nodes x 20 x 20 directions x 500 groups (1.4 GB;
+// HBM floor 248 us), this one 497 us; 18 x 18 x 12 x 12 x 400 216 -> 91 us,
+// 21 x 21 x 13 x 13 x 400 325 -> 235 us.
+constexpr int kRowThreads = 256;
+
+// y[j] = sum_k x[k] S[k][j], four sums at a time; done(j, y[j]) for each j.
+// S: blocked [j / 4][k][j % 4], 64 bytes per two k, requested two such chunks
+// ahead (the scheduling barrier keeps the request there; left to itself the
+// compiler loads all of S and spills scalar registers by the thousand).
+template <int N, typename Done>
+__device__ inline void dst_line(const double* __restrict__ S, const double (&x)[N], Done&& done) {
+    typedef double f64x8 __attribute__((ext_vector_type(8)));
+#pragma unroll 1
+    for (int j = 0; j < N; j += 4) {
+        const f64x8* c = reinterpret_cast<const f64x8*>(S + j * N);
+        f64x8 a = c[0], b = c[1];
+        double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < N; k += 2) {
+            const f64x8 now = a;
+            a = b;
+            if (k + 4 < N) b = c[k / 2 + 2];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                acc[e] = fma(x[k], now[e], acc[e]);
+                acc[e] = fma(x[k + 1], now[4 + e], acc[e]);
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) done(j + e, acc[e]);
+    }
+}
+
+// su, sv: the bases padded to NU x NU and NV x NV, blocked as dst_line reads
+// them.
+template <int NU, int NV>
+__global__ __launch_bounds__(kRowThreads) void angle_rows_kernel(
+    double* __restrict__ F, const double* __restrict__ factors, const double* __restrict__ su,
+    const double* __restrict__ sv, long long planes, int nyz, int Nmu, int Nom, int per_block,
+    const int* __restrict__ top) {
+    extern __shared__ unsigned char lds_raw[];
+    const long long active =
+        top ? min(planes, static_cast<long long>(min(*top, static_cast<int>(planes / nyz) - 1) + 1) * nyz)
+            : planes;
+    const long long p0 = static_cast<long long>(blockIdx.x) * per_block;
+    if (p0 >= active) return;
+    // A plane holds NV rows of pitch values; the rows past Nmu and columns past
+    // Nom are zeros, and stay so: the padded bases make them.
+    constexpr int pitch = NU | 1, plane = NV * pitch;
+    double* X = reinterpret_cast<double*>(lds_raw);
+    const int na = Nmu * Nom;
+    const int np = static_cast<int>(min(static_cast<long long>(per_block), active - p0));
+    const int rows = np * Nmu, cols = np * Nom, n = np * na;
+    double* base = F + p0 * na;
+    if (Nmu < NV || Nom < NU) {
+        for (int e = threadIdx.x; e < np * plane; e += kRowThreads) X[e] = 0.0;
+        __syncthreads();
+    }
+    // coalesced copy of the run: value e sits at column c of row v of a plane;
+    // a step of kRowThreads values is dp planes, dv rows and dc columns
+    const int dr = kRowThreads / Nom, dc = kRowThreads - dr * Nom, dp = dr / Nmu, dv = dr - dp * Nmu;
+    auto each = [&](auto&& f) {
+        const int r = threadIdx.x / Nom;
+        int c = threadIdx.x - r * Nom, p = r / Nmu, v = r - p * Nmu;
+        for (int e = threadIdx.x; e < n; e += kRowThreads) {
+            f(e, p * plane + v * pitch + c);
+            c += dc;
+            v += dv;
+            p += dp;
+            if (c >= Nom) {
+                c -= Nom;
+                ++v;
+            }
+            if (v >= Nmu) {
+                v -= Nmu;
+                ++p;
+            }
+        }
+    };
+    each([&](int e, int at) { X[at] = base[e]; });
+    __syncthreads();
+    auto row_pass = [&] {
+        for (int r = threadIdx.x; r < rows; r += kRowThreads) {
+            const int p = r / Nmu;
+            double* line = X + p * plane + (r - p * Nmu) * pitch;
+            double x[NU];
+#pragma unroll
+            for (int a = 0; a < NU; ++a) x[a] = line[a];
+            dst_line<NU>(su, x, [&](int j, double y) { line[j] = y; });
+        }
+    };
+    row_pass();  // Y[v][mu] = sum_a X[v][a] Su[mu][a]
+    __syncthreads();
+    for (int t = threadIdx.x; t < cols; t += kRowThreads) {
+        const int p = t / Nom, mu = t - p * Nom;
+        const double* C = factors + (p0 + p) / nyz * na + mu;
+        double* line = X + p * plane + mu;
+        double x[NV];
+        auto read = [&] {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) x[v] = line[v * pitch];
+        };
+        // Z[nu][mu] = C[nu][mu] sum_v Sv[nu][v] Y[v][mu], in the column's place
+        read();
+        dst_line<NV>(sv, x, [&](int j, double y) { line[j * pitch] = y * C[min(j, Nmu - 1) * Nom]; });
+        // W[v][mu] = sum_nu Sv[nu][v] Z[nu][mu]
+        read();
+        dst_line<NV>(sv, x, [&](int j, double y) { line[j * pitch] = y; });
+    }
+    __syncthreads();
+    row_pass();  // X'[v][a] = sum_mu W[v][mu] Su[mu][a]
+    __syncthreads();
+    each([&](int e, int at) { base[e] = X[at]; });
+}
+
+// --------------------------------------------------------- vector, wide ---
 
 constexpr int kThreads = 256;
 constexpr int kMaxAngles = 1024;  // Nmu*Nom per plane held in LDS
@@ -521,6 +653,43 @@ void launch_angle_full(T* F, const T* factors, const T* su, const T* sv, int Ng,
     BFPN_REQUIRE(na > 0 && na <= kMaxAngles, "Nmu*Nom must be in [1, 1024]");
     const long long planes = static_cast<long long>(Ng) * nyz;
     if (planes == 0) return;
+    if constexpr (sizeof(T) == 8) {
+        const int widest = std::max(Nmu, Nom);
+        if (widest <= 32) {
+            const int nu = dst_pitch(Nom), nv = dst_pitch(Nmu);
+            // one line per thread in the passes over the longer axis
+            const int per_block = std::max(1, kRowThreads / widest);
+            const size_t lds = sizeof(double) * static_cast<size_t>(per_block) * nv * (nu | 1);
+            const long long blocks = (planes + per_block - 1) / per_block;
+            BFPN_REQUIRE(blocks < (1LL << 31), "too many angular planes");
+            auto go = [&](auto kernel) {
+                BFPN_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             static_cast<int>(lds)));
+                hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kRowThreads),
+                                   lds, s, F, factors, su, sv, planes, nyz, Nmu, Nom, per_block, top);
+            };
+            auto with_nu = [&](auto u) {
+                constexpr int NU = decltype(u)::value;
+                switch (nv) {
+                    case 8: go(&angle_rows_kernel<NU, 8>); break;
+                    case 12: go(&angle_rows_kernel<NU, 12>); break;
+                    case 16: go(&angle_rows_kernel<NU, 16>); break;
+                    case 20: go(&angle_rows_kernel<NU, 20>); break;
+                    default: go(&angle_rows_kernel<NU, 32>); break;
+                }
+            };
+            switch (nu) {
+                case 8: with_nu(std::integral_constant<int, 8>{}); break;
+                case 12: with_nu(std::integral_constant<int, 12>{}); break;
+                case 16: with_nu(std::integral_constant<int, 16>{}); break;
+                case 20: with_nu(std::integral_constant<int, 20>{}); break;
+                default: with_nu(std::integral_constant<int, 32>{}); break;
+            }
+            BFPN_HIP(hipGetLastError());
+            return;
+        }
+    }
     const int per_block = std::max(1, 1024 / na);
     const size_t lds = sizeof(T) * (static_cast<size_t>(Nom) * Nom + static_cast<size_t>(Nmu) * Nmu +
                                     2 * static_cast<size_t>(per_block) * na);

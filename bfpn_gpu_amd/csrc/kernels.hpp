@@ -149,8 +149,11 @@ void launch_transport_half(T* F, const T* omend, int Ny, int Nz, int Ng, int nan
                            double dz, double h, bool preserve_sign, hipStream_t s,
                            const int* top = nullptr);
 
-// CN angular diffusion on the DST-I basis, in place.  factors: Ng*nang (T),
-// su: Nom*Nom, sv: Nmu*Nmu (T).
+// CN angular diffusion on the DST-I basis, in place.  factors: Ng*nang (T);
+// su, sv: the sine bases of Nom and Nmu (T), Nom*Nom and Nmu*Nmu, or, FP64 up to
+// 32 x 32 directions, each padded with zeros to np = dst_pitch() rows and columns
+// and blocked: entry (k, j) at [j / 4][k][j % 4].
+constexpr int dst_pitch(int n) { return n <= 8 ? 8 : n <= 20 ? (n + 3) / 4 * 4 : 32; }
 template <typename T>
 void launch_angle_full(T* F, const T* factors, const T* su, const T* sv, int Ng, int nyz, int Nmu,
                        int Nom, hipStream_t s, const int* top = nullptr);

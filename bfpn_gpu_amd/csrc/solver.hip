@@ -248,6 +248,19 @@ std::string physics_key(const bfpn_grid& g, const bfpn_phys& p, const std::strin
 
 namespace {
 
+// Sine basis of n directions as launch_angle_full<T> reads it for Nmu x Nom.
+template <typename T>
+std::vector<T> dst_basis(int n, int Nmu, int Nom) {
+    const auto s = sine_basis(n);
+    if (sizeof(T) == 4 || std::max(Nmu, Nom) > 32) return cast_vector<T>(s);
+    const int np = dst_pitch(n);
+    std::vector<T> pad(static_cast<size_t>(np) * np, T(0));
+    for (int r = 0; r < n; ++r)
+        for (int c = 0; c < n; ++c)
+            pad[(c / 4 * np + r) * 4 + c % 4] = static_cast<T>(s[r * n + c]);
+    return pad;
+}
+
 enum Phase { kEnergy = 0, kTransport = 1, kAngle = 2, kSource = 3, kDose = 4, kWait = 5 };
 
 // Top group of the secondary source made from a primary state whose top is
@@ -325,8 +338,8 @@ struct Physics final : PhysicsBase {
             upload(om_dev, cast_vector<T>(om));
             upload(factors, cast_vector<T>(angle_factors(sig_tr.data(), g.Ng, g.Nmu, g.Nom, d.du,
                                                          d.dv, d.dt, p.density)));
-            upload(su, cast_vector<T>(sine_basis(g.Nom)));
-            upload(sv, cast_vector<T>(sine_basis(g.Nmu)));
+            upload(su, dst_basis<T>(g.Nom, g.Nmu, g.Nom));
+            upload(sv, dst_basis<T>(g.Nmu, g.Nmu, g.Nom));
             if (std::is_same_v<T, float> &&
                 AnglePlanBuffers::usable(g.Nmu, g.Nom, static_cast<long long>(g.Ng) * nyz))
                 angle_plan.build(g.Nmu, g.Nom, s);
@@ -1627,8 +1640,8 @@ void op_angle(bfpn_workspace* ws, T* F, const double* sig_tr_host, int nyz, int 
         if (mfma) {
             ws->angle_plan.build(Nmu, Nom, s);
         } else {
-            upload(ws->su, cast_vector<T>(sine_basis(Nom)));
-            upload(ws->sv, cast_vector<T>(sine_basis(Nmu)));
+            upload(ws->su, dst_basis<T>(Nom, Nmu, Nom));
+            upload(ws->sv, dst_basis<T>(Nmu, Nmu, Nom));
         }
         ws->angle_key.swap(key);
         ++ws->builds;

@@ -56,3 +56,22 @@ def test_a_plane_that_is_not_finite_spoils_itself_only(gpu, Nmu, Nom, bad):
     spoiled[1, 2] = spoiled[3, 0] = True
     np.testing.assert_array_equal(out[1][~spoiled], out[0][~spoiled])
     assert np.all(np.isnan(out[1][spoiled]))
+
+
+@pytest.mark.parametrize("Nmu,Nom", [(1, 1), (3, 2), (8, 8), (9, 8), (5, 20), (13, 13), (20, 20),
+                                     (21, 3), (20, 17), (32, 32), (33, 31)])
+@pytest.mark.parametrize("nyz,Ng", [(1, 3), (7, 5), (40, 2)])
+def test_fp64_planes_against_the_oracle(gpu, oracle_mod, Nmu, Nom, nyz, Ng):
+    """Lines padded to the kernel's sizes, work-groups part full; 1e-12 of the
+    plane's maximum: four sums of at most 32 products, rounded at 2^-53."""
+    rng = np.random.default_rng(1000 * Nmu + 10 * Nom + nyz)
+    scale = 10.0 ** rng.uniform(-200, 200, (Ng, nyz, 1, 1))
+    F = rng.standard_normal((Ng, nyz, Nmu, Nom)) * scale
+    sig = rng.uniform(0.0, 4.0, Ng)
+    args = (nyz, Ng, Nmu, Nom, 0.2, 0.13, 0.05, 1.2)
+    want = F.ravel().copy()
+    oracle_mod.angle_full(want, sig, *args)
+    d = gpu.DeviceArray(F)
+    gpu.ops.angle_full(d, sig, *args)
+    err = np.abs(d.numpy().reshape(F.shape) - want.reshape(F.shape))
+    assert np.all(err <= 1e-12 * np.abs(F).max(axis=(2, 3), keepdims=True))
