@@ -286,8 +286,8 @@ int beam_top(const BeamFactors& b) {
 template <typename T>
 struct Physics final : PhysicsBase {
     DeviceBuffer coef, dose_w, yzw, om_dev, factors, su, sv, kv, e1, e2, beg, end, qmap, ucoef;
-    DeviceBuffer kcount, klist, need;  // FP64 source: nonzero Kv blocks, groups read
-    DeviceBuffer xmask64;              // FP64: the groups read, as bits (FP32: plan.amask)
+    DeviceBuffer kcount, klist;  // FP64 source: nonzero Kv blocks
+    DeviceBuffer xmask64;        // FP64: the source groups read, as bits (FP32: plan.amask)
     bool legacy = false, lite = false;  // upwind energy model; lite-memory primary step
     double density = 1.0;               // g/cm^3: the IDD and spot-plane scale
     int qcap = -1;                      // highest output group with a source band (-1: none)
@@ -362,7 +362,6 @@ struct Physics final : PhysicsBase {
                     upload(klist, lst);
                     const std::vector<int> nd = source_needed_groups(cnt, ker.beg, ker.end, g.Ng,
                                                                      nang);
-                    upload(need, nd);
                     std::vector<unsigned> bits((g.Ng + 31) / 32, 0u);
                     for (int k = 0; k < g.Ng; ++k)
                         if (nd[k]) bits[k / 32] |= 1u << (k % 32);
@@ -381,7 +380,7 @@ struct Physics final : PhysicsBase {
         return coef.bytes() + dose_w.bytes() + yzw.bytes() + ucoef.bytes() + om_dev.bytes() +
                factors.bytes() +
                su.bytes() + sv.bytes() + kv.bytes() + e1.bytes() + e2.bytes() + beg.bytes() +
-               end.bytes() + qmap.bytes() + kcount.bytes() + klist.bytes() + need.bytes() +
+               end.bytes() + qmap.bytes() + kcount.bytes() + klist.bytes() +
                xmask64.bytes() +
                plan.bytes() +
                angle_plan.h.bytes() +
@@ -875,16 +874,16 @@ private:
             launch_source_mfma(Fp, fp, a1_.as<float>(), a2_.as<float>(), Q, P_->plan.plan,
                                grid.Ng, P_->nyz, P_->nang, s, inputs_read, xt, qm, P_->qcap);
         } else {
-            const int* need = P_->need.template as<int>();
-            launch_source_angular<T>(Fp, fp, P_->kv.template as<T>(), a1_.as<T>(), a2_.as<T>(),
+            const unsigned* rows = P_->xmask64.template as<unsigned>();
+            launch_source_angular(Fp, fp, P_->kv.template as<T>(), a1_.as<T>(), a2_.as<T>(),
                                      grid.Ng, P_->nyz, P_->nang, s, xt,
                                      P_->kcount.template as<int>(), P_->klist.template as<int>(),
-                                     need);
+                                     rows);
             if (inputs_read) BFPN_HIP(hipEventRecord(inputs_read, s));
-            launch_source_energy<T>(a1_.as<T>(), a2_.as<T>(), P_->e1.template as<double>(),
+            launch_source_energy(a1_.as<T>(), a2_.as<T>(), P_->e1.template as<double>(),
                                     P_->e2.template as<double>(), P_->beg.template as<int>(),
                                     P_->end.template as<int>(), Q, grid.Ng, P_->lanes, d.dg, s,
-                                    xt, qm, need);
+                                    xt, qm, rows);
         }
         mark(kSource, array_bytes() * 7, s);  // 2 in, 2 out; 2 in, 1 out
     }
@@ -1177,14 +1176,14 @@ private:
                 launch_source_mfma(Fp, fp, a1_.as<float>(), a2_.as<float>(), Q, P_->plan.plan, Ng, nn,
                                    P_->nang, ss, nullptr, xt, qm, P_->qcap);
             } else {
-                const int* need = P_->need.template as<int>();
-                launch_source_angular<T>(Fp, fp, P_->kv.template as<T>(), a1_.as<T>(), a2_.as<T>(), Ng,
+                const unsigned* rows = P_->xmask64.template as<unsigned>();
+                launch_source_angular(Fp, fp, P_->kv.template as<T>(), a1_.as<T>(), a2_.as<T>(), Ng,
                                          nn, P_->nang, ss, xt, P_->kcount.template as<int>(),
-                                         P_->klist.template as<int>(), need);
-                launch_source_energy<T>(a1_.as<T>(), a2_.as<T>(), P_->e1.template as<double>(),
+                                         P_->klist.template as<int>(), rows);
+                launch_source_energy(a1_.as<T>(), a2_.as<T>(), P_->e1.template as<double>(),
                                         P_->e2.template as<double>(), P_->beg.template as<int>(),
                                         P_->end.template as<int>(), Q, Ng, lanes(k), d.dg, ss, xt, qm,
-                                        need);
+                                        rows);
             }
         };
         double* hist = hist_.as<double>();
@@ -1607,8 +1606,8 @@ void op_source(bfpn_workspace* ws, const T* Fp, const T* fp, T* Q1, const double
         launch_source_mfma(Fp, fp, ws->a1.as<float>(), ws->a2.as<float>(), Q1, ws->plan.plan, Ng,
                            nyz, nang, s);
     } else {
-        launch_source_angular<T>(Fp, fp, kv, ws->a1.as<T>(), ws->a2.as<T>(), Ng, nyz, nang, s);
-        launch_source_energy<T>(ws->a1.as<T>(), ws->a2.as<T>(), e1, e2, beg, end, Q1, Ng,
+        launch_source_angular(Fp, fp, kv, ws->a1.as<T>(), ws->a2.as<T>(), Ng, nyz, nang, s);
+        launch_source_energy(ws->a1.as<T>(), ws->a2.as<T>(), e1, e2, beg, end, Q1, Ng,
                                 static_cast<long long>(nyz) * nang, dg, s);
     }
 }

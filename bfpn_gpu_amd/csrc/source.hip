@@ -12,9 +12,9 @@
 //      band [min beg, max end).
 // FP32 state runs both on the matrix cores in split-BF16 with FP32
 // accumulation (three MFMA issues per tile, ~2^-16 relative per product);
-// the Kv and E operands are split once at set-up.  FP64 state keeps exact
-// FP64 vector kernels (oracle-grade instantiation).  This is the reference's
-// sum regrouped; only rounding order differs.
+// the Kv and E operands are split once at set-up.  FP64 state runs the same two
+// GEMMs on the FP64 matrix cores (oracle-grade instantiation).  This is the
+// reference's sum regrouped; only rounding order differs.
 
 #include "kernels.hpp"
 
@@ -549,173 +549,292 @@ __global__ void split_kernel(const float* __restrict__ src, __bf16* __restrict__
     lo[e] = l;
 }
 
-// ------------------------------------------------------------ FP64 vector --
+// ------------------------------------------------------------ FP64 / MFMA --
+// The same two GEMMs on v_mfma_f64_16x16x4.  The FP64 matrix rate equals the
+// vector rate on this GPU, but a vector kernel cannot issue near it: it reads
+// two LDS operands for every few multiply-adds and its register tiles re-read
+// the A rows once per 16 output groups (measured on 21 x 21 nodes x 20 x 20
+// directions x 500 groups: 2.44 ms angular + 1.49 ms band; here 1.43 + 1.07 ms,
+// the angular one at 80 % of the 68 TFLOP/s that this instruction reaches).
+// Fragments: A lane holds A[i][k], B lane B[k][i], k = lane / 16; D row 4 r +
+// lane / 16, column lane % 16.  Two products share a 16-byte read of the A side
+// by taking k = 2q and 2q + 1 (the order of k is free).
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
 constexpr int kTile = 64;
 constexpr int kDepth = 16;
+constexpr int kDPitch = kDepth + 2;  // doubles per staged row: 16-byte aligned, rows off one bank
 
-template <typename T>
-__global__ __launch_bounds__(256) void source_angular_kernel(const T* __restrict__ Fp,
-                                                             const T* __restrict__ fp,
-                                                             const T* __restrict__ kv,
-                                                             T* __restrict__ A1, T* __restrict__ A2,
-                                                             int nyz, int nang,
-                                                             const int* __restrict__ xtop,
-                                                             const int* __restrict__ kcount,
-                                                             const int* __restrict__ klist,
-                                                             const int* __restrict__ need) {
-    __shared__ T x1s[kDepth][kTile + 1];
-    __shared__ T x2s[kDepth][kTile + 1];
-    __shared__ T ks[kDepth][kTile + 1];
-    const int g = blockIdx.z;
-    if (xtop && g > *xtop) return;  // a zero source group: its A rows are never read
-    if (need && !need[g]) return;   // A rows the banded sum does not read
-    const int m0 = blockIdx.x * kTile;
-    const int s0 = blockIdx.y * kTile;
+__device__ inline f64x4 mma64(double a, double b, f64x4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+// Whether the bit of source group g is set (no mask: every group).
+__device__ inline bool has_group(const unsigned* mask, int g) {
+    return !mask || ((mask[g >> 5] >> (g & 31)) & 1u);
+}
+
+// Angular GEMM.  A work-group: source group g, 64 nodes, 64 directions, both
+// inputs; 4 waves of 32 x 32.  The tiles of one group run on one XCD (they share
+// X[g] and Kv[g] in its L2), groups go round the XCDs.  Per 16-deep K block of
+// Kv with a nonzero entry (kcount / klist; none given: every block) the two X
+// tiles and the Kv tile are staged in LDS, the next block's in registers.
+// VEC: nang % 4 == 0 (16-byte loads of 8-byte aligned pairs).
+template <bool VEC>
+__global__ __launch_bounds__(256) void source_angular_f64(
+    const double* __restrict__ Fp, const double* __restrict__ fp, const double* __restrict__ kv,
+    double* __restrict__ A1, double* __restrict__ A2, int Ng, int nyz, int nang,
+    const int* __restrict__ xtop, const int* __restrict__ kcount, const int* __restrict__ klist,
+    const unsigned* __restrict__ amask) {
+    __shared__ __attribute__((aligned(16))) double xs[2][kTile][kDPitch];
+    // (pitch 72: the rows 2q of the four lane rows alternate between bank halves)
+    __shared__ __attribute__((aligned(16))) double ks[kDepth][kTile + 8];
+    const int mtiles = (nang + kTile - 1) / kTile, stiles = (nyz + kTile - 1) / kTile;
+    const int per_g = mtiles * stiles, seq = blockIdx.x >> 3;
+    const int g = seq / per_g * 8 + (blockIdx.x & 7), rest = seq % per_g;
+    // a zero source group, or one the band GEMM does not read: its A rows stay
+    // unwritten
+    if (g >= Ng || (xtop && g > *xtop) || !has_group(amask, g)) return;
+    const int s0 = rest / mtiles * kTile, mt = rest % mtiles, m0 = mt * kTile;
     const long long plane = static_cast<long long>(g) * nyz * nang;
-    const T* K = kv + static_cast<long long>(g) * nang * nang;
-    const int tx = threadIdx.x & 15;
-    const int ty = threadIdx.x >> 4;
-    T acc1[4][4], acc2[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc1[i][j] = acc2[i][j] = T(0);
-    // With block lists, only the kDepth-deep K blocks where this direction
-    // tile's Kv block has a nonzero entry (the skipped products are zeros).
+    const double* K = kv + static_cast<long long>(g) * nang * nang;
     const int ktiles = (nang + kDepth - 1) / kDepth;
     int nk = ktiles;
     const int* list = nullptr;
     if (kcount) {
-        const long long t = static_cast<long long>(g) * gridDim.x + blockIdx.x;
-        nk = kcount[t];
-        list = klist + t * ktiles;
+        nk = kcount[g * mtiles + mt];
+        list = klist + static_cast<long long>(g * mtiles + mt) * ktiles;
     }
-    for (int kj = 0; kj < nk; ++kj) {
-        const int k0 = (list ? list[kj] : kj) * kDepth;
-        for (int e = threadIdx.x; e < kTile * kDepth; e += 256) {
-            const int kk = e % kDepth, r = e / kDepth;
-            const int s = s0 + r, k = k0 + kk;
-            T v1 = T(0), v2 = T(0);
-            if (s < nyz && k < nang) {
-                const long long idx = plane + static_cast<long long>(s) * nang + k;
-                v1 = Fp[idx] > T(0) ? Fp[idx] : T(0);
-                v2 = fp[idx];
-            }
-            x1s[kk][r] = v1;
-            x2s[kk][r] = v2;
-        }
-        for (int e = threadIdx.x; e < kTile * kDepth; e += 256) {
-            const int c = e % kTile, kk = e / kTile;
-            const int k = k0 + kk, m = m0 + c;
-            ks[kk][c] = (k < nang && m < nang) ? K[static_cast<long long>(k) * nang + m] : T(0);
-        }
-        __syncthreads();
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
+    const int ws = (wave & 1) * 32, wm = (wave >> 1) * 32;
+    // staging: X row lr, columns lk .. + 3; Kv row kr, columns kc .. + 3.  Rows
+    // past nyz read the last one and columns of Kv past nang some other: their
+    // products reach only outputs that are not stored.
+    const int lr = threadIdx.x >> 2, lk = (threadIdx.x & 3) * 4;
+    const int kr = threadIdx.x >> 4, kc = (threadIdx.x & 15) * 4;
+    const long long xrow = plane + static_cast<long long>(min(s0 + lr, nyz - 1)) * nang;
+    double v1[4], v2[4], vk[4];
+    auto load = [&](int k0) {
+        if (VEC) {  // four columns lie inside nang or outside it together
+            const bool in = k0 + lk < nang, kin = k0 + kr < nang;
+            const long long xo = xrow + (in ? k0 + lk : 0);
+            const long long ko =
+                static_cast<long long>(kin ? k0 + kr : 0) * nang + min(m0 + kc, nang - 4);
 #pragma unroll
-        for (int kk = 0; kk < kDepth; ++kk) {
-            T a1[4], a2[4], b[4];
+            for (int h = 0; h < 2; ++h) {
+                const f64x2u a = *reinterpret_cast<const f64x2u*>(Fp + xo + 2 * h);
+                const f64x2u b = *reinterpret_cast<const f64x2u*>(fp + xo + 2 * h);
+                const f64x2u c = *reinterpret_cast<const f64x2u*>(K + ko + 2 * h);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                a1[i] = x1s[kk][ty + 16 * i];
-                a2[i] = x2s[kk][ty + 16 * i];
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = ks[kk][tx + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    acc1[i][j] += a1[i] * b[j];
-                    acc2[i][j] += a2[i] * b[j];
+                for (int e = 0; e < 2; ++e) {
+                    v1[2 * h + e] = in ? a[e] : 0.0;
+                    v2[2 * h + e] = in ? b[e] : 0.0;
+                    vk[2 * h + e] = kin ? c[e] : 0.0;
                 }
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const bool in = k0 + lk + e < nang, kin = k0 + kr < nang;
+                const long long xo = xrow + (in ? k0 + lk + e : 0);
+                v1[e] = in ? Fp[xo] : 0.0;
+                v2[e] = in ? fp[xo] : 0.0;
+                vk[e] = kin ? K[static_cast<long long>(k0 + kr) * nang + min(m0 + kc + e, nang - 1)]
+                            : 0.0;
+            }
+        }
+    };
+    f64x4 acc[2][2][2] = {};  // [input][node tile][direction tile]
+    if (nk > 0) load((list ? list[0] : 0) * kDepth);
+    for (int j = 0; j < nk; ++j) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            *reinterpret_cast<f64x2*>(&xs[0][lr][lk + 2 * h]) =
+                f64x2{v1[2 * h] > 0.0 ? v1[2 * h] : 0.0, v1[2 * h + 1] > 0.0 ? v1[2 * h + 1] : 0.0};
+            *reinterpret_cast<f64x2*>(&xs[1][lr][lk + 2 * h]) = f64x2{v2[2 * h], v2[2 * h + 1]};
+            *reinterpret_cast<f64x2*>(&ks[kr][kc + 2 * h]) = f64x2{vk[2 * h], vk[2 * h + 1]};
+        }
+        __syncthreads();
+        if (j + 1 < nk) load((list ? list[j + 1] : j + 1) * kDepth);
+#pragma unroll
+        for (int h = 0; h < kDepth; h += 8) {
+            f64x2 x[2][2];
+            double b[2][2];  // [k parity][direction tile]
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                x[0][t] = *reinterpret_cast<const f64x2*>(&xs[0][ws + t * 16 + i][h + 2 * q]);
+                x[1][t] = *reinterpret_cast<const f64x2*>(&xs[1][ws + t * 16 + i][h + 2 * q]);
+                b[0][t] = ks[h + 2 * q][wm + t * 16 + i];
+                b[1][t] = ks[h + 2 * q + 1][wm + t * 16 + i];
+            }
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+#pragma unroll
+                for (int in = 0; in < 2; ++in)
+#pragma unroll
+                    for (int st = 0; st < 2; ++st)
+#pragma unroll
+                        for (int dt = 0; dt < 2; ++dt)
+                            acc[in][st][dt] = mma64(x[in][st][e], b[e][dt], acc[in][st][dt]);
         }
         __syncthreads();
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int s = s0 + ty + 16 * i;
-        if (s >= nyz) continue;
+    for (int in = 0; in < 2; ++in) {
+        double* A = in == 0 ? A1 : A2;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int m = m0 + tx + 16 * j;
-            if (m < nang) {
-                const long long idx = plane + static_cast<long long>(s) * nang + m;
-                A1[idx] = acc1[i][j];
-                A2[idx] = acc2[i][j];
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int s = s0 + ws + st * 16 + 4 * r + q;
+                if (s >= nyz) continue;
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt) {
+                    const int m = m0 + wm + dt * 16 + i;
+                    if (m < nang) A[plane + static_cast<long long>(s) * nang + m] = acc[in][st][dt][r];
+                }
             }
-        }
     }
 }
 
-// Banded energy sum, FP64 vector path.  A work-group takes 256 lanes (one
-// per thread) and 16 consecutive output groups, walks the union of their
-// bands once and keeps the 32 sums (E1.A1, E2.A2 per group) in registers, so
-// each A row is read once per 16 output groups rather than once per group.
-// The E rows of the 16 groups are staged through LDS, 128 source groups at a
-// time, and read as broadcasts.  Every sum runs over ascending source groups
-// (a zero weight adds an exact zero), as in the reference's loop.
-constexpr int kEnergyRows = 16;
-constexpr int kEnergyChunk = 128;
+// Banded energy GEMM: Q = dg (K1 . A1 + K2 . A2 / 3).  A work-group: 64 output
+// groups (four 16-row tiles, each over its own band) x 128 lanes, a wave 32
+// lanes.  The weights of 16 source groups at a time pass through LDS, the A
+// rows straight into the waves' B fragments (no two waves share a lane), the
+// next 16 groups' of both in registers.  The group blocks of one lane block run
+// on one XCD.  Taller blocks read an A row fewer times but stage more weights
+// per product: 128 rows x 64 or 128 lanes and 256 x 64 made the source of the
+// grid above 3.12, 2.77 and 4.36 ms against 2.50 ms.
+constexpr int kBand64Tr = 4, kBand64Tc = 2;  // row and lane tiles of a wave
+constexpr int kBand64Rows = 16 * kBand64Tr;
+constexpr int kBand64Lanes = 64 * kBand64Tc;
 
-template <typename T>
-__global__ __launch_bounds__(256) void source_energy_kernel(
-    const T* __restrict__ A1, const T* __restrict__ A2, const double* __restrict__ e1,
+__global__ __launch_bounds__(256) void source_band_f64(
+    const double* __restrict__ A1, const double* __restrict__ A2, const double* __restrict__ e1,
     const double* __restrict__ e2, const int* __restrict__ beg, const int* __restrict__ end,
-    T* __restrict__ Q, int Ng, long long lanes, double dg, const int* __restrict__ xtop,
-    const int* __restrict__ qmap, const int* __restrict__ need) {
-    __shared__ double w1s[kEnergyRows][kEnergyChunk];
-    __shared__ double w2s[kEnergyRows][kEnergyChunk];
-    const int g0 = blockIdx.y * kEnergyRows;
+    double* __restrict__ Q, int Ng, long long lanes, double dg, int lblocks,
+    const int* __restrict__ xtop, const int* __restrict__ qmap, const unsigned* __restrict__ amask) {
+    __shared__ __attribute__((aligned(16))) double es[2][kBand64Rows][kDPitch];
+    __shared__ int bs[kBand64Rows], be[kBand64Rows];
+    constexpr int TR = kBand64Tr, TC = kBand64Tc;
     int kmax = Ng - 1, gmax = Ng - 1;
     if (xtop) {  // groups above the source's top are never read; A rows above kmax are zero
         kmax = max(-1, min(Ng - 1, *xtop));
         gmax = qmap[kmax + 1];
     }
-    if (g0 > gmax) return;
-    const int rows = min(kEnergyRows, gmax - g0 + 1);
-    int kb = Ng, ke = 0;  // union of the rows' bands, below kmax + 1
-    for (int j = 0; j < rows; ++j) {
-        const int b = max(0, beg[g0 + j]), e = min(kmax + 1, end[g0 + j]);
-        if (b < e) {
-            kb = min(kb, b);
-            ke = max(ke, e);
-        }
+    if (gmax < 0) return;
+    const int rblocks = gmax / kBand64Rows + 1, tiles = rblocks * lblocks, n8 = (tiles + 7) & ~7;
+    if (static_cast<int>(blockIdx.x) >= n8) return;
+    const int L = xcd_tile(blockIdx.x, n8);
+    if (L >= tiles) return;
+    const int g0 = L % rblocks * kBand64Rows;
+    const long long n0 = static_cast<long long>(L / rblocks) * kBand64Lanes;
+    if (threadIdx.x < kBand64Rows) {  // bands, cut at the zero A rows; empty: beg >= end
+        const int g = g0 + threadIdx.x;
+        bs[threadIdx.x] = g <= gmax ? max(0, beg[g]) : Ng;
+        be[threadIdx.x] = g <= gmax ? min(kmax + 1, end[g]) : 0;
     }
-    const long long lane = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
-    const bool live = lane < lanes;
-    double q1[kEnergyRows], q2[kEnergyRows];
+    __syncthreads();
+    int tb[TR], te[TR], kb = Ng, ke = 0;
 #pragma unroll
-    for (int j = 0; j < kEnergyRows; ++j) q1[j] = q2[j] = 0.0;
-    for (int c0 = kb; c0 < ke; c0 += kEnergyChunk) {
-        const int cn = min(kEnergyChunk, ke - c0);
-        for (int e = threadIdx.x; e < kEnergyRows * kEnergyChunk; e += 256) {
-            const int j = e / kEnergyChunk, c = e % kEnergyChunk;
-            const bool in = j < rows && c < cn;
-            const long long off = static_cast<long long>(g0 + j) * Ng + c0 + c;
-            w1s[j][c] = in ? e1[off] : 0.0;
-            w2s[j][c] = in ? e2[off] : 0.0;
-        }
-        __syncthreads();
-        if (live) {
-            for (int c = 0; c < cn; ++c) {
-                if (need && !need[c0 + c]) continue;  // A row unwritten; its terms are zeros
-                const long long idx = static_cast<long long>(c0 + c) * lanes + lane;
-                const double a1 = static_cast<double>(A1[idx]);
-                const double a2 = static_cast<double>(A2[idx]);
+    for (int t = 0; t < TR; ++t) {
+        tb[t] = Ng;
+        te[t] = 0;
+        for (int r = 0; r < 16; ++r)
+            if (bs[16 * t + r] < be[16 * t + r]) {
+                tb[t] = min(tb[t], bs[16 * t + r]);
+                te[t] = max(te[t], be[16 * t + r]);
+            }
+        tb[t] = __builtin_amdgcn_readfirstlane(tb[t]);
+        te[t] = __builtin_amdgcn_readfirstlane(te[t]);
+        kb = min(kb, tb[t]);
+        ke = max(ke, te[t]);
+    }
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
+    const int lr = threadIdx.x >> 2, lk = (threadIdx.x & 3) * 4;  // staging: weight row, columns
+    long long col[TC];
 #pragma unroll
-                for (int j = 0; j < kEnergyRows; ++j) {
-                    q1[j] += w1s[j][c] * a1;
-                    q2[j] += w2s[j][c] * a2;
-                }
+    for (int t = 0; t < TC; ++t) col[t] = min(n0 + (wave * TC + t) * 16 + i, lanes - 1);
+    const double dg3 = dg / 3.0;
+    constexpr int TW = kBand64Rows / 64;  // staged weight rows per thread
+    double w1[TW][4], w2[TW][4];
+    double a[2][TC][4];  // [input][lane tile][source groups 2q, 2q + 1 of each half]
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int w = 0; w < TW; ++w)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int g = g0 + 64 * w + lr;
+                const bool in = g < Ng && k0 + lk + e < ke;
+                const long long o = in ? static_cast<long long>(g) * Ng + k0 + lk + e : 0;
+                w1[w][e] = in ? dg * e1[o] : 0.0;
+                w2[w][e] = in ? dg3 * e2[o] : 0.0;
+            }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int k = k0 + 8 * (e >> 1) + 2 * q + (e & 1);
+            const bool in = k < ke && has_group(amask, min(k, Ng - 1));  // else not written, or zero
+            const long long row = static_cast<long long>(in ? k : kb) * lanes;
+#pragma unroll
+            for (int t = 0; t < TC; ++t) {
+                const double x = A1[row + col[t]], y = A2[row + col[t]];
+                a[0][t][e] = in ? x : 0.0;
+                a[1][t][e] = in ? y : 0.0;
             }
         }
+    };
+    f64x4 acc[TR][TC] = {};
+    const int kstart = kb & ~(kDepth - 1);
+    if (kstart < ke) load(kstart);
+    for (int k0 = kstart; k0 < ke; k0 += kDepth) {
+#pragma unroll
+        for (int w = 0; w < TW; ++w)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                *reinterpret_cast<f64x2*>(&es[0][64 * w + lr][lk + 2 * h]) =
+                    f64x2{w1[w][2 * h], w1[w][2 * h + 1]};
+                *reinterpret_cast<f64x2*>(&es[1][64 * w + lr][lk + 2 * h]) =
+                    f64x2{w2[w][2 * h], w2[w][2 * h + 1]};
+            }
+        double now[2][TC][4];
+#pragma unroll
+        for (int in = 0; in < 2; ++in)
+#pragma unroll
+            for (int t = 0; t < TC; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) now[in][t][e] = a[in][t][e];
+        __syncthreads();
+        if (k0 + kDepth < ke) load(k0 + kDepth);
+#pragma unroll
+        for (int mt = 0; mt < TR; ++mt) {
+            if (te[mt] <= tb[mt] || k0 + kDepth <= tb[mt] || k0 >= te[mt]) continue;
+#pragma unroll
+            for (int in = 0; in < 2; ++in)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const f64x2 w =
+                        *reinterpret_cast<const f64x2*>(&es[in][16 * mt + i][8 * h + 2 * q]);
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+#pragma unroll
+                        for (int t = 0; t < TC; ++t)
+                            acc[mt][t] = mma64(w[e], now[in][t][2 * h + e], acc[mt][t]);
+                }
+        }
         __syncthreads();
     }
-    if (!live) return;
 #pragma unroll
-    for (int j = 0; j < kEnergyRows; ++j)
-        if (j < rows)
-            Q[static_cast<long long>(g0 + j) * lanes + lane] =
-                static_cast<T>(dg * (q1[j] + q2[j] / 3.0));
+    for (int mt = 0; mt < TR; ++mt)
+#pragma unroll
+        for (int t = 0; t < TC; ++t) {
+            const long long n = n0 + (wave * TC + t) * 16 + i;
+            if (n >= lanes) continue;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int g = g0 + 16 * mt + 4 * r + q;
+                if (g <= gmax) Q[static_cast<long long>(g) * lanes + n] = acc[mt][t][r];
+            }
+        }
 }
 
 }  // namespace
@@ -844,41 +963,34 @@ void launch_source_mfma(const float* Fp, const float* fp, float* A1, float* A2, 
     BFPN_HIP(hipGetLastError());
 }
 
-template <typename T>
-void launch_source_angular(const T* Fp, const T* fp, const T* kv, T* A1, T* A2, int Ng, int nyz,
-                           int nang, hipStream_t s, const int* xtop, const int* kcount,
-                           const int* klist, const int* need) {
+void launch_source_angular(const double* Fp, const double* fp, const double* kv, double* A1,
+                           double* A2, int Ng, int nyz, int nang, hipStream_t s, const int* xtop,
+                           const int* kcount, const int* klist, const unsigned* amask) {
     if (Ng <= 0 || nyz <= 0 || nang <= 0) return;
-    dim3 grid((nang + kTile - 1) / kTile, (nyz + kTile - 1) / kTile, Ng);
-    hipLaunchKernelGGL(source_angular_kernel<T>, grid, dim3(256), 0, s, Fp, fp, kv, A1, A2, nyz,
-                       nang, xtop, kcount, klist, need);
+    const long long per_g = static_cast<long long>((nang + kTile - 1) / kTile) * ((nyz + kTile - 1) / kTile);
+    const long long blocks = (Ng + 7) / 8 * 8 * per_g;
+    BFPN_REQUIRE(blocks < (1LL << 31), "source GEMM grid too large");
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, Fp, fp, kv,
+                           A1, A2, Ng, nyz, nang, xtop, kcount, klist, amask);
+    };
+    if (nang % 4 == 0) go(&source_angular_f64<true>);
+    else go(&source_angular_f64<false>);
     BFPN_HIP(hipGetLastError());
 }
 
-template <typename T>
-void launch_source_energy(const T* A1, const T* A2, const double* e1, const double* e2,
-                          const int* beg, const int* end, T* Q, int Ng, long long lanes, double dg,
-                          hipStream_t s, const int* xtop, const int* qmap, const int* need) {
+void launch_source_energy(const double* A1, const double* A2, const double* e1, const double* e2,
+                          const int* beg, const int* end, double* Q, int Ng, long long lanes,
+                          double dg, hipStream_t s, const int* xtop, const int* qmap,
+                          const unsigned* amask) {
     if (Ng <= 0 || lanes <= 0) return;
     BFPN_REQUIRE((xtop == nullptr) == (qmap == nullptr), "source tops need both xtop and qmap");
-    dim3 grid(static_cast<unsigned>((lanes + 255) / 256), (Ng + kEnergyRows - 1) / kEnergyRows);
-    hipLaunchKernelGGL(source_energy_kernel<T>, grid, dim3(256), 0, s, A1, A2, e1, e2, beg, end, Q,
-                       Ng, lanes, dg, xtop, qmap, need);
+    const long long lblocks = (lanes + kBand64Lanes - 1) / kBand64Lanes;
+    const long long tiles = lblocks * ((Ng + kBand64Rows - 1) / kBand64Rows);
+    BFPN_REQUIRE(tiles < (1LL << 31) - 8, "source band grid too large");
+    hipLaunchKernelGGL(source_band_f64, dim3(xcd_grid(tiles)), dim3(256), 0, s, A1, A2, e1, e2, beg,
+                       end, Q, Ng, lanes, dg, static_cast<int>(lblocks), xtop, qmap, amask);
     BFPN_HIP(hipGetLastError());
 }
-
-template void launch_source_angular<float>(const float*, const float*, const float*, float*, float*,
-                                           int, int, int, hipStream_t, const int*, const int*,
-                                           const int*, const int*);
-template void launch_source_angular<double>(const double*, const double*, const double*, double*,
-                                            double*, int, int, int, hipStream_t, const int*,
-                                            const int*, const int*, const int*);
-template void launch_source_energy<float>(const float*, const float*, const double*, const double*,
-                                          const int*, const int*, float*, int, long long, double,
-                                          hipStream_t, const int*, const int*, const int*);
-template void launch_source_energy<double>(const double*, const double*, const double*,
-                                           const double*, const int*, const int*, double*, int,
-                                           long long, double, hipStream_t, const int*, const int*,
-                                           const int*);
 
 }  // namespace bfpn
