@@ -10,16 +10,14 @@
 //  * A work-group owns one energy group g and MW consecutive directions m
 //    (the contiguous axis) for the whole (y, z) plane, so no other work-group
 //    reads or writes its data and the update can be written in place.
-//  * Threads own y columns (P of them each) and march along z.  The z window
-//    of psi, psi* and L(psi) stays in registers, and the limited z slopes are
-//    carried from row to row, so each row costs one new z slope per stage.
-//    y neighbours come from LDS rings of 4 rows of psi and 4 rows of psi*.
-//    Step t commits psi row t+2 (prefetched into registers one step earlier),
-//    forms L(psi) and psi* = clip(psi - h L psi) on row t, and writes row t-2:
+//  * Threads own P adjacent y columns and march along z.  The z windows of
+//    psi and psi* stay in registers, and the limited z slopes are carried from
+//    row to row, so each row costs one new z slope per stage.  y neighbours
+//    come from LDS rings of two rows each of psi, psi* and their y slopes.  Step
+//    t forms L(psi) and psi* = clip(psi - h L psi) on row t and writes row t-2:
 //    clip(psi - h/2 (L psi + L psi*)).  One barrier per z step.
 //  * The flow direction is fixed per lane, so only the upwind reconstruction
-//    is formed, in the lane's upwind frame: per stage two limited slopes in y
-//    (the cell's own and its upwind neighbour's) and one in z.
+//    is formed: per stage one limited slope per axis and cell.
 //  * The superbee slope is evaluated without a division:
 //      a = R - C, b = C - L, ab > 0 and |a| >= 1e-10:
 //      slope = sign(a) min(max(|a|, |b|), 2 min(|a|, |b|)),   else 0,
@@ -43,8 +41,18 @@ namespace {
 template <typename T>
 constexpr int max_threads() { return sizeof(T) == 4 ? 1024 : 768; }
 
-// LDS slots per y column (14 used, one pad: an odd pitch in units of MW)
-constexpr int kSlots = 15;
+// Waves per SIMD that the registers have to allow.
+template <typename T, int P>
+constexpr int waves_per_simd() { return sizeof(T) == 4 ? (P == 1 ? 8 : P == 2 ? 5 : 4) : (P == 1 ? 4 : 3); }
+
+// LDS slots of MW values per y column (two rows each of psi, psi* and their
+// y slopes), and the distance of
+// two columns: chosen so that the P columns a thread steps over amount to MW
+// values modulo the banks (P = 1, 2; an odd multiple of MW for P = 3), so the
+// columns that one wave reads fall on distinct banks.
+constexpr int kSlots = 8;
+template <int MW, int P>
+constexpr int column_pitch() { return kSlots * MW + (P == 2 ? MW / 2 : MW); }
 
 // Superbee slope of two differences (either order), without the 1e-10 test:
 //   ab > 0: sign(a) min(max(|a|, |b|), 2 min(|a|, |b|)),  else 0,
@@ -70,65 +78,56 @@ __device__ inline T limited_slope(T a, T b) {
     return fabs(a) < T(1e-10) ? T(0) : superbee(a, b);
 }
 
-// z flux term of a cell in the lane's upwind frame (see divergence):
-// hz (S_c - S_up) + (c - z_up) from the backward differences for wz >= 0 and
-// the negated forward ones otherwise.
-template <typename T>
-__device__ inline T z_term(T dz_b, T dz_f, T dS_b, T dS_f, T hz, bool pz) {
-    return fma(hz, pz ? dS_b : -dS_f, pz ? dz_b : -dz_f);
-}
-
 // Flux divergence at one cell, per axis written in the lane's upwind frame:
 //   w (F(+1/2) - F(-1/2)) / d = (|w| / d) (downwind face - upwind face),
 // where the downwind face is the cell's own reconstruction c + s_down/2 and
-// the upwind face the upwind neighbour's, n + s_up/2, so the difference is
-// (c - n) + (s_down - s_up)/2.  y: from the physical limited slopes of the
-// cell (S_c) and of its upwind neighbour (S_n), the upwind frame's slopes are
-// +-S (superbee is odd and symmetric, and the 1e-10 test goes to the
-// physical forward difference either way), so the y term is
-// (c - n) + hy (S_c - S_n) with hy = +-1/2 the sign of wy.  z: the same with
-// the row window (zm, zc, zp) and the physical slopes of rows -1, 0, +1,
-// given as differences: dz_b = zc - zm, dz_f = zp - zc, dS_b = sz_0 - sz_m,
-// dS_f = sz_p - sz_0 (each is also the other row's difference, so the march
-// forms it once); the upwind terms zc - z_up and sz_0 - sz_up are dz_b, dS_b
-// for wz >= 0 and -dz_f, -dS_f (exact negations) otherwise.  hz = +-1/2 with
-// the sign of wz; cy = |wy| / dy, cz = |wz| / dz.
-// The z term of a row for wz < 0, fma(hz, -dS_f, -dz_f), is the negation of
-// fma(hz, dS_b, dz_b) of the next row (its backward differences are this
-// row's forward ones; rounding to nearest is odd), so the march forms
-// U = fma(hz, dS_f, dz_f) once per row, for the next row's wz >= 0 lanes and
-// this row's other lanes, and selects between U(row) and -U(row + 1).
-template <typename T>
-__device__ inline T divergence(T zc, T near, T S_c, T S_n, T fz, T cy, T cz, T hy) {
-    const T fy = fma(hy, S_c - S_n, zc - near);
-    return cy * fy + cz * fz;
-}
-
-
-// grid: (ceil(nang / MW), Ng), block: MW * R threads (R y columns per pass,
-// P passes: the thread's columns are y = ry + j R).  LDS, stored y-major
-// (column y holds its slots of MW values side by side, pitch 15 MW, odd, so
-// the y columns of one wave fall on distinct banks; a slot is then a constant
-// offset from the column):
-//   slots 0-3   psi rows (row mod 4)        slots 8-11  y slopes of psi rows
-//   slots 4-7   psi* rows (row mod 4)       slots 12-13 y slopes of psi* rows
-// The physical y slope of a row is computed once per cell, two steps before
-// the stage that needs it (after the barrier that publishes the row), kept
-// in a register by its own lane and published in LDS for the downwind
-// neighbour, which reads it instead of recomputing it.
+// the upwind face the upwind neighbour's, n + s_up/2.  The upwind frame's
+// slopes are +-S of the physical limited slopes S (superbee is odd and
+// symmetric, and the 1e-10 test goes to the physical forward difference
+// either way).
+//  y: (c - n) + hy (S_c - S_n), hy = +-1/2 the sign of wy; the physical slope
+//     is formed once per cell and published in LDS for the downwind neighbour.
+//  z: (c - n) + hz (S_c - S_n) from the row window.  For wz < 0 that is the
+//     negation of the next row's value for wz >= 0, so the march forms
+//     U = fma(hz, S(r) - S(r - 1), c(r) - c(r - 1)) once per row r and takes
+//     U(row) or -U(row + 1).
+//
+// grid: (direction chunks x groups, XCD-swizzled), block: MW directions times
+// the y columns, P adjacent columns y = ry P + j per thread, so that inner
+// differences are shared and only the outer neighbours come from LDS.
+//
+// Step t commits psi row t+1 to LDS; after its one barrier it forms the y
+// slopes of psi row t+1 and of psi* row t-1 (for the next step), psi* of row t
+// (predictor) and the result of row t-2 (corrector).  Every ring has two rows:
+// a slot is rewritten one barrier after its last reader.
 //
 // The z march is unrolled by 8: the psi window and the rows in flight share
-// one register ring indexed by row mod 8 (row t+6 is loaded into the slot of
-// row t-2, which step t no longer reads), the other windows are indexed by
-// row mod 4 (slopes by row mod 2), so with the step's phase a compile-time
-// constant, sliding a window is a renaming rather than a chain of moves, a
-// loaded row is never copied (a copy would wait for the load), and the LDS
-// ring slots are immediate offsets.  The corrector needs psi and L(psi) of
-// its row only as psi - h/2 L(psi), kept per row.
+// one register ring indexed by row mod 8 (row t+7 is loaded into the slot of
+// row t-1, which step t no longer reads), so sliding a window is a renaming
+// rather than a chain of moves and a loaded row is never copied (a copy would
+// wait for the load).  Rows past Nz are loaded as copies of row Nz: with them,
+// and with zero slopes carried into rows 0, the clamped stencil at both ends
+// needs no selects.  The first four steps (Start) and the last ones (End)
+// leave out the halves that have no row to work on; those tests are uniform.
+//
+// A corrector adds its two axes' terms in one order up to the step t with
+// t + 13 > Nz and at t = 2, 3 the other way round (Upper and beyond): a choice
+// without meaning that keeps results bit for bit what they have been.
+//
+// What bounds it: vector issue and HBM together (47 vector instructions, 8
+// bytes per cell).  Against a march with four-row rings in LDS (12 LDS
+// accesses per cell instead of 10) whose edge steps did all of their work, one
+// kernel at a time, FP32: 9 x 9 nodes x 49 directions x 500 groups 9.8 -> 8.6
+// us, 11 x 11 x 121 x 500 24.0 -> 17.0, 13 x 13 x 81 x 500 26.6 -> 16.8, 21 x 21
+// x 400 x 500 214 -> 195 (3.6 TB/s), 81 x 81 x 400 x 250 1402 -> 1351 (3.9 TB/s);
+// FP64: 21 x 21 x 400 x 300 293 -> 198, 81 x 81 x 400 x 60 1718 -> 740.
+enum class Part { Start, Inner, Upper, EndLoad, End };
+
 template <typename T, int MW, int P, bool CLIP>
-__global__ __launch_bounds__(max_threads<T>()) void transport_march_kernel(
-    T* __restrict__ F, const T* __restrict__ omend, int Ny, int Nz, int nang, int R, T inv_dy,
-    T inv_dz, T h, int tiles, const int* __restrict__ top) {
+__global__ __launch_bounds__(max_threads<T>())
+__attribute__((amdgpu_waves_per_eu(waves_per_simd<T, P>()))) void transport_march_kernel(
+    T* __restrict__ F, const T* __restrict__ omend, int Ny, int Nz, int nang, T inv_dy, T inv_dz,
+    T h, int tiles, const int* __restrict__ top) {
     extern __shared__ unsigned char lds_raw[];
     const int mchunks = (nang + MW - 1) / MW;
     // Only the groups up to the state's top hold nonzero values (the others
@@ -145,18 +144,19 @@ __global__ __launch_bounds__(max_threads<T>()) void transport_march_kernel(
     if (L >= active) return;
     const int g = L / mchunks;
     T* ring = reinterpret_cast<T*>(lds_raw);
-    constexpr int YP = kSlots * MW;
-    constexpr int kPsi = 0, kPred = 4, kSPsi = 8, kSPred = 12;  // first slot of each ring
+    constexpr int YP = column_pitch<MW, P>();
+    constexpr int kPsi = 0, kPred = 2, kS = 4, kSPred = 6;  // first slot of each ring
 
-    const int mm = threadIdx.x % MW, ry = threadIdx.x / MW;
+    // A thread whose columns would pass Ny takes the last P instead: the ones
+    // it shares with its neighbour get the same values from both.
+    const int mm = threadIdx.x % MW, first = threadIdx.x / MW * P;
+    const int y0 = min(first, Ny + 1 - P);
     const int m0 = (L - g * mchunks) * MW;
     const bool live = m0 + mm < nang;
-    // Lanes past the last direction (and columns past Ny) compute a copy of
-    // the last one from in-bounds addresses, so loads and arithmetic need no
-    // predicate.  Their LDS writes repeat the owner's value at the owner's
-    // slot in the same step (a harmless duplicate), and their global stores
-    // go to an offset past the end of the buffer resource, which the
-    // hardware's range check drops: no store needs a branch.
+    // Lanes past the last direction compute a copy of the last one from
+    // in-bounds addresses, so loads and arithmetic need no predicate; the
+    // global stores of all copies go to an offset past the end of the buffer
+    // resource, which the hardware's range check drops.
     const int m = live ? m0 + mm : nang - 1;
     const T wy = omend[2 * m], wz = omend[2 * m + 1];
     const bool py = wy >= T(0), pz = wz >= T(0);
@@ -173,227 +173,245 @@ __global__ __launch_bounds__(max_threads<T>()) void transport_march_kernel(
 
     unsigned boff[P];  // byte offset of the lane's column in a plane row
     unsigned soff[P];  // the same for stores; kOutside (dropped) for copies
-    int o0[P], o_near[P], o_m[P], o_p[P];  // LDS column: own, upwind, y-1, y+1 (clamped)
-    T win[P][8];    // psi rows t-1 .. t+2 after the commit of step t, then
-                    // rows t+3 .. t+6 in flight (slot: row mod 8)
-    T wpred[P][4];  // psi*, rows t-3 .. t after the predictor of step t
-    T wbase[P][4];  // psi - h/2 L(psi), rows t-2 .. t
-    T wS[P][4];     // own y slope of psi, rows t .. t+2 after step t's slope pass
-    T wSp[P][2];    // own y slope of psi*, rows t-2, t-1 after step t's slope pass
-    T sz[P][2];     // z slopes of psi, rows t-1 and t before step t
-    T szp[P][2];    // z slopes of psi*, rows t-3 and t-2 before step t
-    T uz[P], uzp[P];  // z term U of the row the predictor / corrector works on next
+    T* const own = ring + y0 * YP + mm;  // LDS: the thread's first column,
+    const T *left, *right, *near[P];     // the ones beside it, the upwind ones (clamped)
+    T win[P][8];    // psi rows t .. t+2, then rows t+3 .. t+7 in flight (row mod 8)
+    T wpred[P][4];  // psi*, rows t-2 .. t after the predictor of step t (row mod 4)
+    T wbase[P][4];  // psi - h/2 L(psi), the same rows
+    T sy[P][2], dn[P][2];    // y slope and c - (upwind neighbour) of psi rows t, t+1
+    T syp[P][2], dnp[P][2];  // the same of psi* rows t-2, t-1
+    T sz[P], szp[P];  // z slopes of psi row t and psi* row t-2 before step t
+    T uz[P], uzp[P];  // U of the same rows
+    {
+        auto column = [&](int y) { return ring + min(max(y, 0), Ny) * YP + mm; };
+        left = column(y0 - 1);
+        right = column(y0 + P);
 #pragma unroll
-    for (int j = 0; j < P; ++j) {
-        const int y = ry + j * R;
-        const int yc = min(y, Ny);
-        boff[j] = static_cast<unsigned>((yc * nang + (m - m0)) * sizeof(T));
-        soff[j] = (y <= Ny && live) ? boff[j] : kOutside;
-        auto lo = [&](int yy) { return (min(max(yy, 0), Ny)) * YP + mm; };
-        o0[j] = lo(yc);
-        o_near[j] = lo(py ? yc - 1 : yc + 1);
-        o_m[j] = lo(yc - 1);
-        o_p[j] = lo(yc + 1);
-        const T r0 = bload<T>(Fg, boff[j], 0);
-        const T r1 = bload<T>(Fg, boff[j], zbytes);  // Nz >= 1
-        ring[o0[j] + kPsi * MW] = r0;
-        ring[o0[j] + (kPsi + 1) * MW] = r1;
-        win[j][7] = win[j][0] = r0;  // row -1 clamps to row 0
-        win[j][1] = r1;
-        win[j][6] = T(0);
+        for (int j = 0; j < P; ++j) {
+            const int y = y0 + j;
+            boff[j] = static_cast<unsigned>((y * nang + (m - m0)) * sizeof(T));
+            soff[j] = (y >= first && live) ? boff[j] : kOutside;
+            near[j] = column(py ? y - 1 : y + 1);
 #pragma unroll
-        for (int r = 2; r < 6; ++r)  // rows past Nz: copies of row Nz
-            win[j][r] = bload<T>(Fg, boff[j], static_cast<unsigned>(min(r, Nz)) * zbytes);
-#pragma unroll
-        for (int k = 0; k < 2; ++k) sz[j][k] = szp[j][k] = wSp[j][k] = T(0);  // boundary: 0
-        uz[j] = uzp[j] = T(0);  // (edge steps form their own z terms)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) wpred[j][k] = wbase[j][k] = wS[j][k] = T(0);
+            for (int r = 0; r < 7; ++r)
+                win[j][r] = bload<T>(Fg, boff[j], static_cast<unsigned>(min(r, Nz)) * zbytes);
+            sz[j] = szp[j] = uz[j] = uzp[j] = T(0);
+        }
     }
-    __syncthreads();
-    // y slopes of psi rows 0 and 1 (later rows: two steps ahead, in the march)
+    // y slopes S of a row from its values c and the outer neighbours, into
+    // registers and LDS slot `slot`, and the differences D to the upwind
+    // neighbours.
+    auto slopes = [&](const T (&c)[P], T l, T r, T (&S)[P], T (&D)[P], int slot) {
+        T d[P + 1];
+        d[0] = c[0] - l;
 #pragma unroll
-    for (int j = 0; j < P; ++j) {
+        for (int j = 1; j < P; ++j) d[j] = c[j] - c[j - 1];
+        d[P] = r - c[P - 1];
 #pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            const T* row = ring + (kPsi + r) * MW;
-            const T S = limited_slope(row[o_p[j]] - win[j][r], win[j][r] - row[o_m[j]]);
-            wS[j][r] = S;
-            ring[o0[j] + (kSPsi + r) * MW] = S;
+        for (int j = 0; j < P; ++j) {
+            S[j] = limited_slope(d[j + 1], d[j]);
+            D[j] = py ? d[j] : -d[j + 1];
+            own[j * YP + slot * MW] = S[j];
+        }
+    };
+    {
+#pragma unroll
+        for (int j = 0; j < P; ++j) own[j * YP + kPsi * MW] = win[j][0];
+        __syncthreads();
+        T c[P], S[P], D[P];
+#pragma unroll
+        for (int j = 0; j < P; ++j) c[j] = win[j][0];
+        slopes(c, left[kPsi * MW], right[kPsi * MW], S, D, kS);
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            sy[j][0] = S[j];
+            dn[j][0] = D[j];
         }
     }
 
-    // Step t (phase k8 = t mod 8, k = t mod 4): commit psi row t+2; slopes of
-    // psi row t+2 and psi* row t-1; predictor on row t; corrector on row t-2.
-    // Every step runs the same branch-free code; near the ends of the march
-    // (EDGE) selects apply the clamped rows and the boundary slopes, and the
-    // global store is skipped (uniformly) before row 0 and past row Nz.  Past
-    // the last row the predictor works on clamped copies and its result is
-    // replaced by the clamp; steps past Nz+2 (padding the last block) store
-    // nothing.
-    auto step = [&](int t, auto phase, auto edge) {
+    auto step = [&](int t, auto phase, auto part) {
         constexpr int k8 = decltype(phase)::value;  // t mod 8
-        constexpr int k = k8 & 3;
-        constexpr bool E = decltype(edge)::value;
-        const int rc = t + 2;  // commit psi row t+2 (LDS ring slot of row t-2)
-        {
-            T* crow = ring + (kPsi + ((k + 2) & 3)) * MW;
+        constexpr int k2 = k8 & 1, k4 = k8 & 3;
+        constexpr Part S = decltype(part)::value;
+        constexpr bool E = S == Part::End || S == Part::EndLoad;
+        if (E && t > Nz + 2) return;
+        const bool do_slope = !E || t + 1 <= Nz;
+        const bool do_pred = !E || t <= Nz;
+        const bool do_slopep = S == Part::Start ? k8 >= 1 : !E || t <= Nz + 1;
+        const bool do_corr = S != Part::Start || k8 >= 2;
+        if (do_slope)
 #pragma unroll
-            for (int j = 0; j < P; ++j) {
-                if (E && rc > Nz) win[j][(k8 + 2) & 7] = win[j][(k8 + 1) & 7];
-                crow[o0[j]] = win[j][(k8 + 2) & 7];
-            }
-        }
+            for (int j = 0; j < P; ++j) own[j * YP + (kPsi + (k2 ^ 1)) * MW] = win[j][(k8 + 1) & 7];
         __syncthreads();
         // Keep each step's arithmetic after its barrier: moved earlier, the z
         // differences of later rows would wait for rows still in flight.
         __builtin_amdgcn_sched_barrier(0);
-        {
-            // row t+6 into the register slot of row t-2: four rows in flight
-            const unsigned so = static_cast<unsigned>(E ? min(t + 6, Nz) : t + 6) * zbytes;
+        // row t+7 into the register slot of row t-1: five rows in flight
+        if (S != Part::End) {
+            const unsigned so = static_cast<unsigned>(min(t + 7, Nz)) * zbytes;
 #pragma unroll
-            for (int j = 0; j < P; ++j) win[j][(k8 + 6) & 7] = bload<T>(Fg, boff[j], so);
+            for (int j = 0; j < P; ++j) win[j][(k8 + 7) & 7] = bload<T>(Fg, boff[j], so);
         }
-        // LDS reads of the step, issued together: y neighbours of psi row t+2
-        // and psi* row t-1 (their slopes), upwind value and slope of psi row t
-        // (predictor) and psi* row t-2 (corrector)
-        T a_m[P], a_p[P], b_m[P], b_p[P], pn[P], pS[P], cn_[P], cS[P];
-        {
-            const T* psi2 = ring + (kPsi + ((k + 2) & 3)) * MW;    // psi row t+2
-            const T* prd1 = ring + (kPred + ((k + 3) & 3)) * MW;   // psi* row t-1
-            const T* psi0 = ring + (kPsi + k) * MW;                // psi row t
-            const T* sps0 = ring + (kSPsi + k) * MW;               // its slopes
-            const T* prd2 = ring + (kPred + ((k + 2) & 3)) * MW;   // psi* row t-2
-            const T* spd2 = ring + (kSPred + (k & 1)) * MW;        // its slopes
+        // LDS reads of the step, issued together
+        T al = T(0), ar = T(0), bl = T(0), br = T(0), en[P], cn[P];
+        if (do_slope) {
+            al = left[(kPsi + (k2 ^ 1)) * MW];
+            ar = right[(kPsi + (k2 ^ 1)) * MW];
+        }
+        if (do_slopep) {
+            bl = left[(kPred + (k2 ^ 1)) * MW];
+            br = right[(kPred + (k2 ^ 1)) * MW];
+        }
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            en[j] = do_pred ? near[j][(kS + k2) * MW] : T(0);
+            cn[j] = do_corr ? near[j][(kSPred + k2) * MW] : T(0);
+        }
+        if (do_slope) {  // y slopes of psi row t+1
+            T c[P], S[P], D[P];
+#pragma unroll
+            for (int j = 0; j < P; ++j) c[j] = win[j][(k8 + 1) & 7];
+            slopes(c, al, ar, S, D, kS + (k2 ^ 1));
 #pragma unroll
             for (int j = 0; j < P; ++j) {
-                a_m[j] = psi2[o_m[j]];
-                a_p[j] = psi2[o_p[j]];
-                b_m[j] = prd1[o_m[j]];
-                b_p[j] = prd1[o_p[j]];
-                pn[j] = psi0[o_near[j]];
-                pS[j] = sps0[o_near[j]];
-                cn_[j] = prd2[o_near[j]];
-                cS[j] = spd2[o_near[j]];
+                sy[j][k2 ^ 1] = S[j];
+                dn[j][k2 ^ 1] = D[j];
             }
         }
-        {  // y slopes of psi row t+2 and psi* row t-1, published for step t+2
-            T* sp2 = ring + (kSPsi + ((k + 2) & 3)) * MW;
-            T* sd1 = ring + (kSPred + ((k + 1) & 1)) * MW;
+        if (do_slopep) {  // y slopes of psi* row t-1
+            T c[P], S[P], D[P];
+#pragma unroll
+            for (int j = 0; j < P; ++j) c[j] = wpred[j][(k4 + 3) & 3];
+            slopes(c, bl, br, S, D, kSPred + (k2 ^ 1));
 #pragma unroll
             for (int j = 0; j < P; ++j) {
-                const T c2 = win[j][(k8 + 2) & 7], c1 = wpred[j][(k + 3) & 3];
-                const T S2 = limited_slope(a_p[j] - c2, c2 - a_m[j]);
-                const T S1 = limited_slope(b_p[j] - c1, c1 - b_m[j]);
-                wS[j][(k + 2) & 3] = S2;
-                wSp[j][(k + 1) & 1] = S1;
-                sp2[o0[j]] = S2;
-                sd1[o0[j]] = S1;
+                syp[j][k2 ^ 1] = S[j];
+                dnp[j][k2 ^ 1] = D[j];
             }
         }
-        {  // predictor on row t
-            T* prow = ring + (kPred + k) * MW;
+        if (do_pred) {  // predictor on row t
 #pragma unroll
             for (int j = 0; j < P; ++j) {
-                const T zm = win[j][(k8 + 7) & 7], zc = win[j][k8], zp = win[j][(k8 + 1) & 7];
-                const T dz_b = zc - zm, dz_f = zp - zc;
-                const T s_next = limited_slope(win[j][(k8 + 2) & 7] - zp, dz_f);
-                const T sz_m = sz[j][(k + 1) & 1], sz_0 = sz[j][k & 1];
-                const T dS_f = s_next - sz_0;
-                const T un = fma(hz, dS_f, dz_f);  // U of row t+1
-                const T fz = E ? z_term(dz_b, dz_f, sz_0 - sz_m, dS_f, hz, pz) : (pz ? uz[j] : -un);
+                const T c = win[j][k8], up = win[j][(k8 + 1) & 7];
+                const T dz = up - c;
+                const T s = limited_slope(win[j][(k8 + 2) & 7] - up, dz);
+                const T un = fma(hz, s - sz[j], dz);  // U of row t+1
+                const T fy = fma(hy, sy[j][k2] - en[j], dn[j][k2]), fz = pz ? uz[j] : -un;
+                const T L0 = fma(cy, fy, cz * fz);
+                sz[j] = s;
                 uz[j] = un;
-                const T L0 = divergence(zc, pn[j], wS[j][k], pS[j], fz, cy, cz, hy);
-                T v = zc - h * L0;
+                T v = c - h * L0;
                 if (CLIP) v = fmax(v, T(0));
-                prow[o0[j]] = v;
-                sz[j][(k + 1) & 1] = s_next;
-                wbase[j][k] = zc - hh * L0;
-                wpred[j][k] = (!E || t <= Nz) ? v : wpred[j][(k + 3) & 3];  // past Nz: row Nz
-                if (E && k == 0) wpred[j][3] = t == 0 ? v : wpred[j][3];  // row -1: row 0
+                wbase[j][k4] = c - hh * L0;
+                // rows past Nz: copies of row Nz
+                wpred[j][k4] = S == Part::Start && k8 >= 2 && t > Nz ? wpred[j][(k4 + 3) & 3] : v;
+                own[j * YP + (kPred + k2) * MW] = v;
             }
+        } else {
+#pragma unroll
+            for (int j = 0; j < P; ++j) wpred[j][k4] = wpred[j][(k4 + 3) & 3];  // past Nz: row Nz
         }
-        {  // corrector on row t-2, written in place
-            const unsigned so = static_cast<unsigned>(E ? max(t - 2, 0) : t - 2) * zbytes;
-            const bool real = !E || (t >= 2 && t <= Nz + 2);
+        if (do_corr) {  // corrector on row t-2, written in place
+            const unsigned so = static_cast<unsigned>(t - 2) * zbytes;
 #pragma unroll
             for (int j = 0; j < P; ++j) {
-                const T zm = wpred[j][(k + 1) & 3], zc = wpred[j][(k + 2) & 3],
-                        zp = wpred[j][(k + 3) & 3];
-                const T dz_b = zc - zm, dz_f = zp - zc;
-                const T s_next = limited_slope(wpred[j][k] - zp, dz_f);
-                const T sz_m = szp[j][(k + 1) & 1], sz_0 = szp[j][k & 1];
-                const T dS_f = s_next - sz_0;
-                const T un = fma(hz, dS_f, dz_f);  // U of row t-1
-                const T fz = E ? z_term(dz_b, dz_f, sz_0 - sz_m, dS_f, hz, pz) : (pz ? uzp[j] : -un);
-                const T L1 = divergence(zc, cn_[j], wSp[j][k & 1], cS[j], fz, cy, cz, hy);
-                T v = wbase[j][(k + 2) & 3] - hh * L1;
+                const T c = wpred[j][(k4 + 2) & 3], up = wpred[j][(k4 + 3) & 3];
+                const T dz = up - c;
+                const T s = limited_slope(wpred[j][k4] - up, dz);
+                const T un = fma(hz, s - szp[j], dz);  // U of row t-1
+                const T fy = fma(hy, syp[j][k2] - cn[j], dnp[j][k2]), fz = pz ? uzp[j] : -un;
+                const T L1 = S == Part::Inner ? fma(cy, fy, cz * fz) : fma(cz, fz, cy * fy);
+                szp[j] = s;
+                uzp[j] = un;
+                T v = wbase[j][(k4 + 2) & 3] - hh * L1;
                 if (CLIP) v = fmax(v, T(0));
-                if (real) bstore(v, Fg, soff[j], so);
-                const T s_kept = (!E || t >= 2) ? s_next : T(0);  // rows <= 0: boundary
-                szp[j][(k + 1) & 1] = s_kept;
-                // the next row's U from the slope kept for it (at edge steps the
-                // kept slope may be the boundary's 0)
-                uzp[j] = E ? fma(hz, s_kept - sz_0, dz_f) : un;
+                bstore(v, Fg, soff[j], so);
             }
         }
     };
     // four steps from t0, t0 mod 8 = B
-    auto block = [&](int t0, auto base, auto edge) {
+    auto block = [&](int t0, auto base, auto part) {
         constexpr int B = decltype(base)::value;
-        step(t0, std::integral_constant<int, B>{}, edge);
-        step(t0 + 1, std::integral_constant<int, B + 1>{}, edge);
-        step(t0 + 2, std::integral_constant<int, B + 2>{}, edge);
-        step(t0 + 3, std::integral_constant<int, B + 3>{}, edge);
+        step(t0, std::integral_constant<int, B>{}, part);
+        step(t0 + 1, std::integral_constant<int, B + 1>{}, part);
+        step(t0 + 2, std::integral_constant<int, B + 2>{}, part);
+        step(t0 + 3, std::integral_constant<int, B + 3>{}, part);
     };
     using I0 = std::integral_constant<int, 0>;
     using I4 = std::integral_constant<int, 4>;
-    block(0, I0{}, std::true_type{});
+    using Start = std::integral_constant<Part, Part::Start>;
+    using Inner = std::integral_constant<Part, Part::Inner>;
+    using Upper = std::integral_constant<Part, Part::Upper>;
+    using EndLoad = std::integral_constant<Part, Part::EndLoad>;
+    using End = std::integral_constant<Part, Part::End>;
+    // One straight path: alternatives for the last blocks that join again cost
+    // 20 to 40 registers.
+    block(0, I0{}, Start{});
     int t0 = 4;
-    // interior: 2 <= t and t + 6 <= Nz for all eight steps
     for (; t0 + 13 <= Nz; t0 += 8) {
-        block(t0, I4{}, std::false_type{});
-        block(t0 + 4, I0{}, std::false_type{});
+        block(t0, I4{}, Inner{});
+        block(t0 + 4, I0{}, Inner{});
     }
-    for (; t0 <= Nz + 2; t0 += 8) {
-        block(t0, I4{}, std::true_type{});
-        if (t0 + 4 > Nz + 2) break;
-        block(t0 + 4, I0{}, std::true_type{});
+    for (; t0 + 8 <= Nz; t0 += 8) {  // (at most once)
+        block(t0, I4{}, Upper{});
+        block(t0 + 4, I0{}, Upper{});
     }
+    // at most 10 steps are left; rows up to Nz + 2 are loaded in the first three
+    block(t0, I4{}, EndLoad{});
+    block(t0 + 4, I0{}, End{});
+    step(t0 + 8, I4{}, End{});
+    step(t0 + 9, std::integral_constant<int, 5>{}, End{});
 }
 
 struct MarchShape {
-    int MW, P, R, threads;
+    int MW, P, threads;
 };
 
-// Launch shape, the first of (MW, P) = (16, 1), (16, 2), (8, 2), (8, 3)
-// whose work-group covers the plane and whose LDS rings fit the
-// 160 KB of a CU.  Measured on MI355X (FP32, 400 directions): 16 directions
-// per work-group beat 32 (smaller groups pack the CU's wave slots better:
-// 235 vs 248 us at 21 x 21 nodes) and 8 (64-byte row segments: 3.41 vs
-// 3.57 ms at 81 x 81 nodes with two columns per thread).  At 81 x 81 nodes
-// the (16, 2) shape runs one work-group per CU; 12 or 8 directions with one
-// column per thread fit two, but their 48- and 32-byte row segments cost
-// more than the occupancy gains (3.30 and 3.78 vs 2.52 ms per launch).
-MarchShape march_shape(int Ny1, size_t elem) {
-    const int max_t = elem == 4 ? max_threads<float>() : max_threads<double>();
-    constexpr int cand[4][2] = {{16, 1}, {16, 2}, {8, 2}, {8, 3}};
-    for (const auto& c : cand) {
-        const int MW = c[0], P = c[1];
-        if (static_cast<long long>(max_t / MW) * P < Ny1) continue;
-        if (static_cast<size_t>(kSlots) * Ny1 * MW * elem > 160 * 1024) continue;
-        const int R0 = (Ny1 + P - 1) / P;
-        const int threads = (MW * R0 + 63) / 64 * 64;
-        return MarchShape{MW, P, threads / MW, threads};
+// Launch shape of a plane of Ny1 columns.
+// FP32: 16 directions per work-group (8: 32-byte row segments, 253 against
+// 195 us at 21 x 21 nodes x 400 directions x 500 groups) with the P of the
+// fewest wave columns (waves x P): P adjacent columns share their differences,
+// but a thread's lanes past the plane cost P columns each.  Ties go to the
+// smaller P (13 x 13 x 81 x 500: 17.0 us with one column per thread, 18.8 with
+// two; whole 21 x 21 beam steps measured the same with either).  81 x 81 nodes
+// x 400 x 250: P = 3, 1.35 ms, against 1.38 with 2.
+// FP64: a thread's windows allow four waves per SIMD, so what counts is how
+// many of a CU's 16 wave slots whole work-groups fill: 24 directions (two
+// work-groups of 8 waves) at 21 columns, 198 us for 400 x 300, against 252 with
+// 16 (two of 6) and 206 with 8; 8 directions at 81 columns.  Wider planes take
+// several columns per thread.
+MarchShape march_shape(int Ny1, int nang, size_t elem) {
+    auto threads_of = [&](int MW, int P) { return (MW * ((Ny1 + P - 1) / P) + 63) / 64 * 64; };
+    MarchShape best{0, 0, 0};
+    if (elem == 8) {
+        double least = 0.0;
+        for (const int MW : {16, 24, 8}) {
+            const int threads = threads_of(MW, 1), waves = threads / 64;
+            if (threads > max_threads<double>()) continue;
+            const double cost = static_cast<double>((nang + MW - 1) / MW) / (16 / waves);
+            if (best.MW && cost >= least) continue;
+            least = cost;
+            best = MarchShape{MW, 1, threads};
+        }
+        for (int P = 2; P <= 3 && !best.MW; ++P)
+            if (threads_of(8, P) <= max_threads<double>()) best = MarchShape{8, P, threads_of(8, P)};
+        return best;
     }
-    return MarchShape{0, 0, 0, 0};
+    constexpr int cand[][2] = {{16, 1}, {16, 2}, {16, 3}, {8, 3}};
+    for (const auto& c : cand) {
+        const int MW = c[0], P = c[1], threads = threads_of(MW, P);
+        if (Ny1 < P || threads > max_threads<float>()) continue;
+        if (best.MW && (MW < best.MW || threads * P >= best.threads * best.P)) continue;
+        best = MarchShape{MW, P, threads};
+    }
+    return best;
 }
 
 template <typename T, int MW, int P>
-void launch_march(T* F, const T* omend, int Ny, int Nz, int Ng, int nang, const MarchShape& sh,
-                  double dy, double dz, double h, bool preserve_sign, hipStream_t s,
-                  const int* top) {
-    const size_t lds = sizeof(T) * kSlots * static_cast<size_t>(Ny + 1) * MW;
+void launch_march(T* F, const T* omend, int Ny, int Nz, int Ng, int nang, int threads, double dy,
+                  double dz, double h, bool preserve_sign, hipStream_t s, const int* top) {
+    BFPN_REQUIRE(Ny + 1 >= P, "a transport thread needs its P columns");
+    const size_t lds = sizeof(T) * column_pitch<MW, P>() * (Ny + 1);
     BFPN_REQUIRE(lds <= 160 * 1024, "transport plane too wide for the LDS rings");
     const long long tiles = static_cast<long long>((nang + MW - 1) / MW) * Ng;
     BFPN_REQUIRE(tiles < (1LL << 31) - 8, "transport grid too large");
@@ -402,7 +420,7 @@ void launch_march(T* F, const T* omend, int Ny, int Nz, int Ng, int nang, const 
         BFPN_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                      hipFuncAttributeMaxDynamicSharedMemorySize,
                                      static_cast<int>(lds)));
-        hipLaunchKernelGGL(kernel, grid, dim3(sh.threads), lds, s, F, omend, Ny, Nz, nang, sh.R,
+        hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, s, F, omend, Ny, Nz, nang,
                            static_cast<T>(1.0 / dy), static_cast<T>(1.0 / dz), static_cast<T>(h),
                            static_cast<int>(tiles), top);
     };
@@ -421,21 +439,27 @@ void launch_transport_half(T* F, const T* omend, int Ny, int Nz, int Ng, int nan
                            const int* top) {
     if (Ng <= 0 || nang <= 0) return;
     BFPN_REQUIRE(Ny >= 1 && Nz >= 1, "transport needs Ny, Nz >= 1");
-    const MarchShape sh = march_shape(Ny + 1, sizeof(T));
-    // the LDS holds 15 slots of MW values per y column: 15 * (Ny+1) * 8 * elem <= 160 KB
-    BFPN_REQUIRE(sh.MW > 0, sizeof(T) == 4 ? "transport supports at most 341 y nodes in FP32"
-                                           : "transport supports at most 170 y nodes in FP64");
+    BFPN_REQUIRE(Ny + 1 <= (sizeof(T) == 4 ? 341 : 170),
+                 sizeof(T) == 4 ? "transport supports at most 341 y nodes in FP32"
+                                : "transport supports at most 170 y nodes in FP64");
     // one group's block is addressed with 32-bit byte offsets
     BFPN_REQUIRE(static_cast<long long>(Ny + 1) * (Nz + 1) * nang * sizeof(T) < (1LL << 31),
                  "transport needs (Ny+1)(Nz+1)*Nmu*Nom values of one energy group below 2 GiB");
-#define BFPN_MARCH(MW_, P_)                                                                    \
-    if (sh.MW == MW_ && sh.P == P_)                                                            \
-        return launch_march<T, MW_, P_>(F, omend, Ny, Nz, Ng, nang, sh, dy, dz, h, preserve_sign, \
-                                        s, top)
+    const MarchShape sh = march_shape(Ny + 1, nang, sizeof(T));
+#define BFPN_MARCH(MW_, P_)                                                                   \
+    if (sh.MW == MW_ && sh.P == P_)                                                           \
+        return launch_march<T, MW_, P_>(F, omend, Ny, Nz, Ng, nang, sh.threads, dy, dz, h,     \
+                                        preserve_sign, s, top)
     BFPN_MARCH(16, 1);
-    BFPN_MARCH(16, 2);
-    BFPN_MARCH(8, 2);
     BFPN_MARCH(8, 3);
+    if constexpr (sizeof(T) == 4) {
+        BFPN_MARCH(16, 2);
+        BFPN_MARCH(16, 3);
+    } else {
+        BFPN_MARCH(24, 1);
+        BFPN_MARCH(8, 1);
+        BFPN_MARCH(8, 2);
+    }
 #undef BFPN_MARCH
     throw Error(BFPN_E_INVALID, "no transport launch shape for this plane");
 }

@@ -1,0 +1,34 @@
+"""The transport march at the edges of its parts and launch shapes.
+
+Marches of 2 to 23 rows end in every place of the unrolled blocks; the column
+counts give 1, 2 and 3 columns per thread (the last thread sharing columns with
+its neighbour or not) and, in FP64, 8, 16 and 24 directions per work-group.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# the bounds of one transport application against the oracle (test_gpu_ops.py)
+TOL = {np.float64: 1e-12, np.float32: 5e-5}
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("Ny,Nz,nang", [(13, n, 17) for n in range(1, 23)] +
+                         [(1, 9, 5), (2, 5, 23), (10, 11, 49), (20, 12, 25), (21, 8, 24), (33, 6, 40),
+                          (66, 4, 9), (81, 13, 33), (95, 3, 8), (96, 5, 3), (169, 2, 3)])
+def test_against_the_oracle(gpu, oracle_mod, Ny, Nz, nang, dtype):
+    rng = np.random.default_rng(1000 * Ny + Nz)
+    Ng, n = 3, (Ny + 1) * (Nz + 1) * nang
+    F = rng.standard_normal(Ng * n)
+    F[::5] = np.round(F[::5])  # ties and flat runs
+    F = F.astype(dtype).astype(np.float64)
+    om = rng.uniform(-0.9, 0.9, 2 * nang)
+    d_om = gpu.DeviceArray(om.astype(np.float64))
+    for preserve in (True, False):
+        ref = F.copy()
+        dF = gpu.DeviceArray(F.astype(dtype))
+        gpu.ops.transport_half(dF, d_om, Ny, Nz, Ng, nang, 0.2, 0.3, 0.05, preserve)
+        oracle_mod.transport_half(ref, om, Ny, Nz, Ng, nang, 0.2, 0.3, 0.05, preserve)
+        err = np.abs(dF.numpy().astype(np.float64) - ref).max() / np.abs(ref).max()
+        assert err <= TOL[dtype]
