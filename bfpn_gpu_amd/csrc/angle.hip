@@ -55,11 +55,12 @@ namespace {
 // the bases' columns (stage 1, the repeated ones as zeros) and rows (stage 4,
 // where both lanes compute the same value) in that order, angle_column().
 template <int MT, int NT, bool V4>
-__global__ __launch_bounds__(256) void angle_mfma_kernel(float* __restrict__ F,
+__global__ __launch_bounds__(256) void angle_mfma_kernel(float* __restrict__ F_, float* __restrict__ f_,
                                                          const float* __restrict__ factors,
                                                          AnglePlan plan, int planes, int per_wave,
                                                          int nyz, int Nmu, int Nom, float one,
                                                          const int* __restrict__ top) {
+    float* const F = blockIdx.y ? f_ : F_;  // the second array of a launch over two
     // Only the planes of groups up to the state's top are nonzero (the
     // others stay zero): the first `active` planes, shared out evenly over
     // the grid's waves; blocks without any exit before touching LDS.
@@ -269,11 +270,12 @@ __global__ __launch_bounds__(256) void angle_mfma_kernel(float* __restrict__ F,
 // floor 42 us) 104 -> 44 us, 11 x 11 (26.7 M) 114 -> 47, 10 x 10 (12.8 M)
 // 61 -> 33, 7 x 7 (2 M, launch included) 23 -> 13.
 template <bool PM2, bool PN2, bool VEC>
-__global__ __launch_bounds__(256) void angle_small_kernel(float* __restrict__ F,
+__global__ __launch_bounds__(256) void angle_small_kernel(float* __restrict__ F_, float* __restrict__ f_,
                                                           const float* __restrict__ factors,
                                                           AnglePlan plan, int planes, int per_wave,
                                                           int nyz, int Nmu, int Nom, float one,
                                                           const int* __restrict__ top) {
+    float* const F = blockIdx.y ? f_ : F_;  // the second array of a launch over two
     constexpr int NPN = PN2 ? 2 : 1, P = (PM2 ? 2 : 1) * NPN;  // planes per tile
     const int Ng = planes / nyz;
     const int active = top ? min(planes, (min(*top, Ng - 1) + 1) * nyz) : planes;
@@ -603,7 +605,7 @@ __global__ __launch_bounds__(kThreads) void angle_kernel(T* __restrict__ F,
 }  // namespace
 
 void launch_angle_mfma(float* F, const float* factors, const AnglePlan& plan, int Ng, int nyz,
-                       int Nmu, int Nom, hipStream_t s, const int* top) {
+                       int Nmu, int Nom, hipStream_t s, const int* top, float* f) {
     BFPN_REQUIRE(Nmu >= 1 && Nom >= 1 && Nmu <= 32 && Nom <= 32, "MFMA DST needs Nmu, Nom <= 32");
     const long long planes = static_cast<long long>(Ng) * nyz;
     if (planes == 0) return;
@@ -620,7 +622,7 @@ void launch_angle_mfma(float* F, const float* factors, const AnglePlan& plan, in
     int per_wave = 0;
     auto go = [&](auto kernel, int planes_per_tile) {
         const int blocks = shape(planes_per_tile, per_wave);
-        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, s, F, factors, plan,
+        hipLaunchKernelGGL(kernel, dim3(blocks, f ? 2 : 1), dim3(256), 0, s, F, f, factors, plan,
                            static_cast<int>(planes), per_wave, nyz, Nmu, Nom, 1.0f, top);
     };
     const bool vec = Nom >= 4;

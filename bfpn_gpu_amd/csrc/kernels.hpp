@@ -145,7 +145,7 @@ void launch_source_energy(const double* A1, const double* A2, const double* e1, 
 template <typename T>
 void launch_transport_half(T* F, const T* omend, int Ny, int Nz, int Ng, int nang, double dy,
                            double dz, double h, bool preserve_sign, hipStream_t s,
-                           const int* top = nullptr);
+                           const int* top = nullptr, T* f = nullptr);
 
 // CN angular diffusion on the DST-I basis, in place.  factors: Ng*nang (T);
 // su, sv: the sine bases of Nom and Nmu (T), Nom*Nom and Nmu*Nmu, or, FP64 up to
@@ -182,8 +182,10 @@ constexpr int angle_column(int k, int n) {
 // K slot 8q + 4u + r of a chained MFMA operand <-> matrix index 16u + 4q + r.
 constexpr int chain_index(int slot) { return 16 * ((slot & 7) >> 2) + 4 * (slot >> 3) + (slot & 3); }
 // FP32 DST on the matrix cores (Nmu, Nom <= 32), in place.
+// f: a second array of the same sizes in the same launch (optional).
 void launch_angle_mfma(float* F, const float* factors, const AnglePlan& plan, int Ng, int nyz,
-                       int Nmu, int Nom, hipStream_t s, const int* top = nullptr);
+                       int Nmu, int Nom, hipStream_t s, const int* top = nullptr,
+                       float* f = nullptr);
 
 // Eq.24 dose of (F+F1, f+f1) into per-block partials (count = dose_blocks()).
 template <typename T>
@@ -201,8 +203,10 @@ void launch_dose_coefs(const double* S, const double* sigma, const double* en, d
 void launch_yz_weights(int Ny, int Nz, bool trapezoidal, double* out, hipStream_t s);
 
 // out[slot] = scale * sum(a[0:na]) + scale * sum(b[0:nb])  (b may be null), one block.
+// With out2, also *out2 = scale2 sum(a2[0:na]), in the same launch.
 void launch_finish_sum(const double* a, int na, const double* b, int nb, double scale, double* out,
-                       hipStream_t s);
+                       hipStream_t s, const double* a2 = nullptr, double scale2 = 0.0,
+                       double* out2 = nullptr);
 // *out = ((0 + v[0]) + v[1]) + ... + v[n-1], in that order.
 void launch_sum_in_order(const double* v, int n, double* out, hipStream_t s);
 

@@ -82,8 +82,16 @@ __global__ __launch_bounds__(kBlock) void dose_kernel(const T* __restrict__ F,
 
 __global__ __launch_bounds__(1024) void finish_sum_kernel(const double* __restrict__ a, int na,
                                                           const double* __restrict__ b, int nb,
-                                                          double scale, double* __restrict__ out) {
+                                                          double scale, double* __restrict__ out,
+                                                          const double* __restrict__ a2,
+                                                          double scale2, double* __restrict__ out2) {
     __shared__ double lds[1024];
+    if (blockIdx.x == 1) {
+        a = a2;
+        b = nullptr;
+        scale = scale2;
+        out = out2;
+    }
     double s = 0.0;
     for (int k = threadIdx.x; k < na; k += 1024) s += a[k];
     if (b)
@@ -353,8 +361,9 @@ void launch_dose(const T* F, const T* f, const T* F1, const T* f1, const DoseCoe
 }
 
 void launch_finish_sum(const double* a, int na, const double* b, int nb, double scale, double* out,
-                       hipStream_t s) {
-    hipLaunchKernelGGL(finish_sum_kernel, dim3(1), dim3(1024), 0, s, a, na, b, nb, scale, out);
+                       hipStream_t s, const double* a2, double scale2, double* out2) {
+    hipLaunchKernelGGL(finish_sum_kernel, dim3(out2 ? 2 : 1), dim3(1024), 0, s, a, na, b, nb, scale,
+                       out, a2, scale2, out2);
     BFPN_HIP(hipGetLastError());
 }
 

@@ -862,6 +862,41 @@ private:
         mark(kAngle, array_bytes() * 2, s);
     }
 
+    // Both arrays of a species (psi^2 keeps its sign), in one launch where one
+    // array's is short: below kPairBytes a launch lasts less than about 60 us
+    // and its first and last waves, and the gap to the next, are a good part of
+    // it (whole 9 x 9 node solve 57.0 -> 52.8 ms, 40 steps on the default grid
+    // 16.2 -> 15.4 ms; a 21 x 21 node beam, 353 MB an array, measured the same
+    // either way).
+    static constexpr size_t kPairBytes = size_t(64) << 20;
+    bool paired() const { return cells * sizeof(T) < kPairBytes; }
+    void transport_both(int species, bool preserve_sign, hipStream_t s) {
+        const int w = 2 * species;
+        if (!paired()) {
+            transport(w, preserve_sign, s);
+            transport(w + 1, true, s);
+            return;
+        }
+        launch_transport_half<T>(cur_[w], P_->om_dev.template as<T>(), grid.Ny, grid.Nz, grid.Ng,
+                                 P_->nang, d.dy, d.dz, 0.5 * d.dt, preserve_sign, s,
+                                 cur_top(species), cur_[w + 1]);
+        mark(kTransport, array_bytes() * 4, s);
+    }
+    void angle_both(int species, hipStream_t s) {
+        const int w = 2 * species;
+        if constexpr (std::is_same_v<T, float>) {
+            if (paired() && P_->angle_plan.plan.su_h) {
+                launch_angle_mfma(cur_[w], P_->factors.template as<float>(), P_->angle_plan.plan,
+                                  grid.Ng, P_->nyz, grid.Nmu, grid.Nom, s, cur_top(species),
+                                  cur_[w + 1]);
+                mark(kAngle, array_bytes() * 4, s);
+                return;
+            }
+        }
+        angle(w, s);
+        angle(w + 1, s);
+    }
+
     // Secondary source Q from the primary state (Fp, fp) on stream s;
     // `inputs_read` (optional) is recorded on s once (Fp, fp) have been read
     // (after the angular GEMM).
@@ -951,18 +986,9 @@ private:
             energy(0, nullptr, nullptr, false, sp, sweep_tops(0, -1, -1, -1));
         }
         if (!phys.energy_only) {
-            if (!phys.no_transport) {
-                transport(0, preserve_primary, sp);
-                transport(1, true, sp);
-            }
-            if (!phys.no_angle) {
-                angle(0, sp);
-                angle(1, sp);
-            }
-            if (!phys.no_transport) {
-                transport(0, preserve_primary, sp);
-                transport(1, true, sp);
-            }
+            if (!phys.no_transport) transport_both(0, preserve_primary, sp);
+            if (!phys.no_angle) angle_both(0, sp);
+            if (!phys.no_transport) transport_both(0, preserve_primary, sp);
         }
         if (last) {
             energy(0, nullptr, pp, true, sp, sweep_tops(0, -1, -1, n));
@@ -984,8 +1010,8 @@ private:
         double* hist = hist_.as<double>();
         auto finish = [&](int m, bool with_secondary) {  // IDD and proxy of step m
             double* pm = partial_p_.as<double>() + (m & 3) * 2 * eb;
-            launch_finish_sum(pm, eb, with_secondary ? ps : nullptr, eb, scale, hist + m, ss);
-            launch_finish_sum(pm + eb, eb, nullptr, 0, d.dg, hist + hist_cap_ + m, ss);
+            launch_finish_sum(pm, eb, with_secondary ? ps : nullptr, eb, scale, hist + m, ss, pm + eb,
+                              d.dg, hist + hist_cap_ + m);
             mark(kDose, 0.0, ss);
         };
         const bool sec = secondary && n > 0;
@@ -1000,12 +1026,9 @@ private:
             } else {
                 energy(1, Q, nullptr, false, ss, sweep_tops(1, n, -1, -1));
             }
-            transport(2, false, ss);  // secondary psi^1 is always clipped
-            transport(3, true, ss);
-            angle(2, ss);
-            angle(3, ss);
-            transport(2, false, ss);
-            transport(3, true, ss);
+            transport_both(1, false, ss);  // secondary psi^1 is always clipped
+            angle_both(1, ss);
+            transport_both(1, false, ss);
             if (last) {
                 energy(1, Q, ps, false, ss, sweep_tops(1, n, -1, -1));
                 finish(n, true);

@@ -124,10 +124,9 @@ __device__ inline T limited_slope(T a, T b) {
 enum class Part { Start, Inner, Upper, EndLoad, End };
 
 template <typename T, int MW, int P, bool CLIP>
-__global__ __launch_bounds__(max_threads<T>())
-__attribute__((amdgpu_waves_per_eu(waves_per_simd<T, P>()))) void transport_march_kernel(
-    T* __restrict__ F, const T* __restrict__ omend, int Ny, int Nz, int nang, T inv_dy, T inv_dz,
-    T h, int tiles, const int* __restrict__ top) {
+__device__ __forceinline__ void transport_march(T* __restrict__ F, const T* __restrict__ omend, int Ny, int Nz,
+                                       int nang, T inv_dy, T inv_dz, T h, int tiles,
+                                       const int* __restrict__ top) {
     extern __shared__ unsigned char lds_raw[];
     const int mchunks = (nang + MW - 1) / MW;
     // Only the groups up to the state's top hold nonzero values (the others
@@ -363,6 +362,28 @@ __attribute__((amdgpu_waves_per_eu(waves_per_simd<T, P>()))) void transport_marc
     step(t0 + 9, std::integral_constant<int, 5>{}, End{});
 }
 
+// Which arrays a launch marches and how: one with or without the clip, or a
+// species' two in one launch (blockIdx.y): psi^1 with or without, psi^2 without.
+enum class Arrays { Clipped, Signed, ClippedSigned, SignedSigned };
+
+template <typename T, int MW, int P, Arrays A>
+__global__ __launch_bounds__(max_threads<T>())
+__attribute__((amdgpu_waves_per_eu(waves_per_simd<T, P>()))) void transport_march_kernel(
+    T* __restrict__ F, T* __restrict__ f, const T* __restrict__ omend, int Ny, int Nz, int nang,
+    T inv_dy, T inv_dz, T h, int tiles, const int* __restrict__ top) {
+    if constexpr (A == Arrays::Clipped) {
+        transport_march<T, MW, P, true>(F, omend, Ny, Nz, nang, inv_dy, inv_dz, h, tiles, top);
+    } else if constexpr (A == Arrays::ClippedSigned) {
+        if (blockIdx.y == 0)
+            transport_march<T, MW, P, true>(F, omend, Ny, Nz, nang, inv_dy, inv_dz, h, tiles, top);
+        else
+            transport_march<T, MW, P, false>(f, omend, Ny, Nz, nang, inv_dy, inv_dz, h, tiles, top);
+    } else {
+        T* const X = A == Arrays::SignedSigned && blockIdx.y ? f : F;
+        transport_march<T, MW, P, false>(X, omend, Ny, Nz, nang, inv_dy, inv_dz, h, tiles, top);
+    }
+}
+
 struct MarchShape {
     int MW, P, threads;
 };
@@ -408,26 +429,30 @@ MarchShape march_shape(int Ny1, int nang, size_t elem) {
 }
 
 template <typename T, int MW, int P>
-void launch_march(T* F, const T* omend, int Ny, int Nz, int Ng, int nang, int threads, double dy,
+void launch_march(T* F, T* f, const T* omend, int Ny, int Nz, int Ng, int nang, int threads, double dy,
                   double dz, double h, bool preserve_sign, hipStream_t s, const int* top) {
     BFPN_REQUIRE(Ny + 1 >= P, "a transport thread needs its P columns");
     const size_t lds = sizeof(T) * column_pitch<MW, P>() * (Ny + 1);
     BFPN_REQUIRE(lds <= 160 * 1024, "transport plane too wide for the LDS rings");
     const long long tiles = static_cast<long long>((nang + MW - 1) / MW) * Ng;
     BFPN_REQUIRE(tiles < (1LL << 31) - 8, "transport grid too large");
-    const dim3 grid(static_cast<unsigned>((tiles + 7) / 8 * 8));
+    const dim3 grid(static_cast<unsigned>((tiles + 7) / 8 * 8), f ? 2 : 1);
     auto go = [&](auto kernel) {
         BFPN_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                      hipFuncAttributeMaxDynamicSharedMemorySize,
                                      static_cast<int>(lds)));
-        hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, s, F, omend, Ny, Nz, nang,
+        hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, s, F, f, omend, Ny, Nz, nang,
                            static_cast<T>(1.0 / dy), static_cast<T>(1.0 / dz), static_cast<T>(h),
                            static_cast<int>(tiles), top);
     };
-    if (preserve_sign)
-        go(&transport_march_kernel<T, MW, P, false>);
+    if (f && preserve_sign)
+        go(&transport_march_kernel<T, MW, P, Arrays::SignedSigned>);
+    else if (f)
+        go(&transport_march_kernel<T, MW, P, Arrays::ClippedSigned>);
+    else if (preserve_sign)
+        go(&transport_march_kernel<T, MW, P, Arrays::Signed>);
     else
-        go(&transport_march_kernel<T, MW, P, true>);
+        go(&transport_march_kernel<T, MW, P, Arrays::Clipped>);
     BFPN_HIP(hipGetLastError());
 }
 
@@ -436,7 +461,7 @@ void launch_march(T* F, const T* omend, int Ny, int Nz, int Ng, int nang, int th
 template <typename T>
 void launch_transport_half(T* F, const T* omend, int Ny, int Nz, int Ng, int nang, double dy,
                            double dz, double h, bool preserve_sign, hipStream_t s,
-                           const int* top) {
+                           const int* top, T* f) {
     if (Ng <= 0 || nang <= 0) return;
     BFPN_REQUIRE(Ny >= 1 && Nz >= 1, "transport needs Ny, Nz >= 1");
     BFPN_REQUIRE(Ny + 1 <= (sizeof(T) == 4 ? 341 : 170),
@@ -448,7 +473,7 @@ void launch_transport_half(T* F, const T* omend, int Ny, int Nz, int Ng, int nan
     const MarchShape sh = march_shape(Ny + 1, nang, sizeof(T));
 #define BFPN_MARCH(MW_, P_)                                                                   \
     if (sh.MW == MW_ && sh.P == P_)                                                           \
-        return launch_march<T, MW_, P_>(F, omend, Ny, Nz, Ng, nang, sh.threads, dy, dz, h,     \
+        return launch_march<T, MW_, P_>(F, f, omend, Ny, Nz, Ng, nang, sh.threads, dy, dz, h,     \
                                         preserve_sign, s, top)
     BFPN_MARCH(16, 1);
     BFPN_MARCH(8, 3);
@@ -465,8 +490,8 @@ void launch_transport_half(T* F, const T* omend, int Ny, int Nz, int Ng, int nan
 }
 
 template void launch_transport_half<float>(float*, const float*, int, int, int, int, double, double,
-                                           double, bool, hipStream_t, const int*);
+                                           double, bool, hipStream_t, const int*, float*);
 template void launch_transport_half<double>(double*, const double*, int, int, int, int, double,
-                                            double, double, bool, hipStream_t, const int*);
+                                            double, double, bool, hipStream_t, const int*, double*);
 
 }  // namespace bfpn

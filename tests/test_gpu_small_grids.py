@@ -62,3 +62,21 @@ def test_paired_sweeps_at_group_and_lane_edges(gpu, oracle_mod, Ng, over, stragg
                 a, r = one.state(k), ref.state(k)
                 np.testing.assert_array_equal(a, many.state(k))
                 assert np.abs(a - r).max() <= tol * max(np.abs(r).max(), 1e-300)
+
+
+@pytest.mark.parametrize("over", [dict(Ny=5, Nz=7, Nmu=7, Nom=6), dict(Ny=9, Nz=4, Nmu=11, Nom=11),
+                                  dict(Ny=4, Nz=5, Nmu=18, Nom=17), dict(Ny=15, Nz=2, Nmu=3, Nom=9)])
+@pytest.mark.parametrize("no_clip", [0, 1])
+def test_both_arrays_in_one_launch(gpu, oracle_mod, over, no_clip):
+    """Whole steps on grids whose transport and angular launches take both
+    arrays of a species, the primary's psi^1 clipped or signed."""
+    c = small_case(Ng=60, Lg=31.08, energy=20.0, flags=dict(no_spatial_clipping=no_clip), **over)
+    ref = oracle_mod.Solver(c)
+    ref.advance(4)
+    for precision, tol in ((gpu.FP64, 1e-10), (gpu.FP32, 2e-4)):
+        with gpu.Solver(c, precision) as s:
+            s.advance(4)
+            np.testing.assert_allclose(s.history()[0], ref.history()[0], rtol=tol)
+            for k in range(4):
+                a, r = s.state(k), ref.state(k)
+                assert np.abs(a - r).max() <= tol * max(np.abs(r).max(), 1e-300)
