@@ -34,6 +34,25 @@ namespace {
 __device__ inline int xcd_tile(int b, int grid) { return (b & 7) * (grid >> 3) + (b >> 3); }
 inline int xcd_grid(long long tiles) { return static_cast<int>((tiles + 7) / 8 * 8); }
 
+// 16-byte accesses at any multiple of 4 bytes.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ inline void load8(const float* p, float (&v)[8]) {
+    const f32x4u a = *reinterpret_cast<const f32x4u*>(p), b = *reinterpret_cast<const f32x4u*>(p + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[e] = a[e];
+        v[4 + e] = b[e];
+    }
+}
+// p[0..3], of which the first n (any n) exist; the others read as zero.
+__device__ inline float4 load4_upto(const float* p, long long n) {
+    if (n >= 4) {
+        const f32x4u v = *reinterpret_cast<const f32x4u*>(p);
+        return make_float4(v[0], v[1], v[2], v[3]);
+    }
+    return make_float4(n > 0 ? p[0] : 0.f, n > 1 ? p[1] : 0.f, n > 2 ? p[2] : 0.f, 0.f);
+}
+
 // Angular GEMM.  Logical tile = (g, 64 transverse nodes, 64 directions); the
 // 7 x 7 tiles of one source group g share X[g] and Kv[g] through one L2.
 // Kv is thresholded (at 20 x 20 directions, water 230 MeV, 58 % of its
@@ -43,7 +62,10 @@ inline int xcd_grid(long long tiles) { return static_cast<int>((tiles + 7) / 8 *
 // work-group stages a 64(s) x 32(m') tile of both inputs -- split into BF16
 // hi/lo once -- and the matching 64(m) x 32(m') tile of the pre-split
 // transposed Kv in LDS; the next step's global loads are in flight while the
-// matrix cores work on the current one.  VEC: nang % 8 == 0 (16-byte loads).
+// matrix cores work on the current one.  VEC: nang % 8 == 0 (every row starts
+// at 16 bytes and holds whole vectors); otherwise vectors at 4-byte alignment,
+// value by value only where a row ends inside one (whole source at 11 x 11
+// directions: 53,361 lanes x 500 groups 315 -> 194 us, value by value before).
 constexpr int kKPitch = 40;  // bf16 per LDS row (32 + 8 pad)
 
 template <bool VEC>
@@ -106,6 +128,9 @@ __global__ __launch_bounds__(256) void source_angular_mfma(const float* __restri
             v1[4] = a1.x; v1[5] = a1.y; v1[6] = a1.z; v1[7] = a1.w;
             v2[0] = b0.x; v2[1] = b0.y; v2[2] = b0.z; v2[3] = b0.w;
             v2[4] = b1.x; v2[5] = b1.y; v2[6] = b1.z; v2[7] = b1.w;
+        } else if (srow < nyz && k0 + lk + 8 <= nang) {
+            load8(Fp + base, v1);
+            load8(fp + base, v2);
         } else {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
@@ -189,6 +214,8 @@ __global__ __launch_bounds__(256) void source_angular_mfma(const float* __restri
                 const long long idx = plane + static_cast<long long>(sidx) * nang + m;
                 if (VEC) {  // nang % 8 == 0: m + 3 < nang and 16-byte aligned
                     *reinterpret_cast<float4*>(A + idx) = make_float4(v[0], v[1], v[2], v[3]);
+                } else if (m + 4 <= nang) {
+                    *reinterpret_cast<f32x4u*>(A + idx) = f32x4u{v[0], v[1], v[2], v[3]};
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
@@ -286,15 +313,8 @@ __global__ __launch_bounds__(256) void source_band_mfma(
                     r2[j] = *reinterpret_cast<const float4*>(A2 + idx);
                 }
             } else {
-                float a[4], b[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const bool in = has && ln + e < lanes;
-                    a[e] = in ? A1[idx + e] : 0.f;
-                    b[e] = in ? A2[idx + e] : 0.f;
-                }
-                r1[j] = make_float4(a[0], a[1], a[2], a[3]);
-                r2[j] = make_float4(b[0], b[1], b[2], b[3]);
+                r1[j] = load4_upto(A1 + idx, has ? lanes - ln : 0);
+                r2[j] = load4_upto(A2 + idx, has ? lanes - ln : 0);
             }
         }
         // rows g_base .. g_base+63 < erows and columns k0 .. k0+31 < ngp
@@ -416,10 +436,7 @@ __global__ __launch_bounds__(512, 4) void source_band_march(
                 ra[j] = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (has && ln < lanes) ra[j] = *reinterpret_cast<const float4*>(A + idx);
             } else {
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = has && ln + e < lanes ? A[idx + e] : 0.f;
-                ra[j] = make_float4(v[0], v[1], v[2], v[3]);
+                ra[j] = load4_upto(A + idx, has ? lanes - ln : 0);
             }
         }
         const int2 w = steps[k];  // live tiles [x, y]
@@ -904,6 +921,15 @@ void launch_split(const float* src, __bf16* hi, __bf16* lo, long long n, hipStre
     BFPN_HIP(hipGetLastError());
 }
 
+// The march needs enough lane blocks: with at most one work-group per CU each
+// walks all source steps by itself while half the wave slots stay empty, and
+// the tiles over output groups, which re-read A rows from the caches, are faster.
+// Whole source, 500 groups: 3,969 lanes 91 us by the march and 31 by tiles,
+// 14,641 123 and 58, 32,400 126 and 115; 176,400 619 and 656.
+static bool source_marches(const SourcePlan& plan, long long lanes) {
+    return plan.march && lanes > 256LL * kMarchLanes;
+}
+
 void launch_source_mfma(const float* Fp, const float* fp, float* A1, float* A2, float* Q,
                         const SourcePlan& plan, int Ng, int nyz, int nang, hipStream_t s,
                         hipEvent_t inputs_read, const int* xtop, const int* qmap, int q_rows) {
@@ -929,7 +955,7 @@ void launch_source_mfma(const float* Fp, const float* fp, float* A1, float* A2, 
     }
     if (inputs_read) BFPN_HIP(hipEventRecord(inputs_read, s));
     const long long lanes = static_cast<long long>(nyz) * nang;
-    if (plan.march) {
+    if (source_marches(plan, lanes)) {
         const long long lb = (lanes + kMarchLanes - 1) / kMarchLanes;
         BFPN_REQUIRE(lb < (1LL << 31) - 8, "source band grid too large");
         const int gm = xcd_grid(lb);
