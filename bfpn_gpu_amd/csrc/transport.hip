@@ -119,7 +119,7 @@ __device__ inline T limited_slope(T a, T b) {
 // accesses per cell instead of 10) whose edge steps did all of their work, one
 // kernel at a time, FP32: 9 x 9 nodes x 49 directions x 500 groups 9.8 -> 8.6
 // us, 11 x 11 x 121 x 500 24.0 -> 17.0, 13 x 13 x 81 x 500 26.6 -> 16.8, 21 x 21
-// x 400 x 500 214 -> 195 (3.6 TB/s), 81 x 81 x 400 x 250 1402 -> 1351 (3.9 TB/s);
+// x 400 x 500 214 -> 195 (3.6 TB/s), 81 x 81 x 400 x 250 1402 -> 1376 (3.8 TB/s);
 // FP64: 21 x 21 x 400 x 300 293 -> 198, 81 x 81 x 400 x 60 1718 -> 740.
 enum class Part { Start, Inner, Upper, EndLoad, End };
 
@@ -389,13 +389,14 @@ struct MarchShape {
 };
 
 // Launch shape of a plane of Ny1 columns.
-// FP32: 16 directions per work-group (8: 32-byte row segments, 253 against
-// 195 us at 21 x 21 nodes x 400 directions x 500 groups) with the P of the
-// fewest wave columns (waves x P): P adjacent columns share their differences,
-// but a thread's lanes past the plane cost P columns each.  Ties go to the
-// smaller P (13 x 13 x 81 x 500: 17.0 us with one column per thread, 18.8 with
-// two; whole 21 x 21 beam steps measured the same with either).  81 x 81 nodes
-// x 400 x 250: P = 3, 1.35 ms, against 1.38 with 2.
+// FP32: the first of (directions, columns per thread) = (16, 1), (16, 2),
+// (8, 2), (8, 3) whose work-group fits.  8 directions are 32-byte row segments
+// (254 against 195 us at 21 x 21 nodes x 400 directions x 500 groups), so they
+// are for the widest planes.  More columns per thread than needed share more
+// differences but leave fewer waves per SIMD: two cost 18.8 against 17.0 us at
+// 13 x 13 x 81 x 500 and the same over whole 21 x 21 beam steps; three at 81 x 81
+// were 2 % faster alone (1.35 ms, x 400 x 250) and slowed the whole step, where
+// the other stream's kernels run beside them, from 47.6 to 50.7 ms.
 // FP64: a thread's windows allow four waves per SIMD, so what counts is how
 // many of a CU's 16 wave slots whole work-groups fill: 24 directions (two
 // work-groups of 8 waves) at 21 columns, 198 us for 400 x 300, against 252 with
@@ -418,12 +419,10 @@ MarchShape march_shape(int Ny1, int nang, size_t elem) {
             if (threads_of(8, P) <= max_threads<double>()) best = MarchShape{8, P, threads_of(8, P)};
         return best;
     }
-    constexpr int cand[][2] = {{16, 1}, {16, 2}, {16, 3}, {8, 3}};
+    constexpr int cand[][2] = {{16, 1}, {16, 2}, {8, 2}, {8, 3}};
     for (const auto& c : cand) {
         const int MW = c[0], P = c[1], threads = threads_of(MW, P);
-        if (Ny1 < P || threads > max_threads<float>()) continue;
-        if (best.MW && (MW < best.MW || threads * P >= best.threads * best.P)) continue;
-        best = MarchShape{MW, P, threads};
+        if (threads <= max_threads<float>()) return MarchShape{MW, P, threads};
     }
     return best;
 }
@@ -476,14 +475,13 @@ void launch_transport_half(T* F, const T* omend, int Ny, int Nz, int Ng, int nan
         return launch_march<T, MW_, P_>(F, f, omend, Ny, Nz, Ng, nang, sh.threads, dy, dz, h,     \
                                         preserve_sign, s, top)
     BFPN_MARCH(16, 1);
+    BFPN_MARCH(8, 2);
     BFPN_MARCH(8, 3);
     if constexpr (sizeof(T) == 4) {
         BFPN_MARCH(16, 2);
-        BFPN_MARCH(16, 3);
     } else {
         BFPN_MARCH(24, 1);
         BFPN_MARCH(8, 1);
-        BFPN_MARCH(8, 2);
     }
 #undef BFPN_MARCH
     throw Error(BFPN_E_INVALID, "no transport launch shape for this plane");
