@@ -43,7 +43,9 @@ constexpr int max_threads() { return sizeof(T) == 4 ? 1024 : 768; }
 
 // Waves per SIMD that the registers have to allow.
 template <typename T, int P>
-constexpr int waves_per_simd() { return sizeof(T) == 4 ? (P == 1 ? 8 : P == 2 ? 5 : 4) : (P == 1 ? 4 : 3); }
+constexpr int waves_per_simd() {
+    return sizeof(T) == 4 ? (P == 1 ? 8 : P == 2 ? 5 : 4) : (P == 1 ? 4 : 3);
+}
 
 // LDS slots of MW values per y column (two rows each of psi, psi* and their
 // y slopes), and the distance of
@@ -124,9 +126,9 @@ __device__ inline T limited_slope(T a, T b) {
 enum class Part { Start, Inner, Upper, EndLoad, End };
 
 template <typename T, int MW, int P, bool CLIP>
-__device__ __forceinline__ void transport_march(T* __restrict__ F, const T* __restrict__ omend, int Ny, int Nz,
-                                       int nang, T inv_dy, T inv_dz, T h, int tiles,
-                                       const int* __restrict__ top) {
+__device__ __forceinline__ void transport_march(T* __restrict__ F, const T* __restrict__ omend,
+                                                int Ny, int Nz, int nang, T inv_dy, T inv_dz, T h,
+                                                int tiles, const int* __restrict__ top) {
     extern __shared__ unsigned char lds_raw[];
     const int mchunks = (nang + MW - 1) / MW;
     // Only the groups up to the state's top hold nonzero values (the others
@@ -415,9 +417,8 @@ MarchShape march_shape(int Ny1, int nang, size_t elem) {
             least = cost;
             best = MarchShape{MW, 1, threads};
         }
-        for (int P = 2; P <= 3 && !best.MW; ++P)
-            if (threads_of(8, P) <= max_threads<double>()) best = MarchShape{8, P, threads_of(8, P)};
-        return best;
+        // (two columns per thread reach 192 columns; the limit is 170)
+        return best.MW ? best : MarchShape{8, 2, threads_of(8, 2)};
     }
     constexpr int cand[][2] = {{16, 1}, {16, 2}, {8, 2}, {8, 3}};
     for (const auto& c : cand) {
@@ -476,9 +477,9 @@ void launch_transport_half(T* F, const T* omend, int Ny, int Nz, int Ng, int nan
                                         preserve_sign, s, top)
     BFPN_MARCH(16, 1);
     BFPN_MARCH(8, 2);
-    BFPN_MARCH(8, 3);
     if constexpr (sizeof(T) == 4) {
         BFPN_MARCH(16, 2);
+        BFPN_MARCH(8, 3);
     } else {
         BFPN_MARCH(24, 1);
         BFPN_MARCH(8, 1);

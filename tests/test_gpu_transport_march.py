@@ -1,7 +1,7 @@
 """The transport march at the edges of its parts and launch shapes.
 
 Marches of 2 to 23 rows end in every place of the unrolled blocks; the column
-counts give 1, 2 and 3 columns per thread (the last thread sharing columns with
+counts give one column per thread or more (the last thread sharing columns with
 its neighbour or not) and, in FP64, 8, 16 and 24 directions per work-group.
 """
 import numpy as np
