@@ -36,6 +36,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "angle_operands.hpp"
 #include "device.hpp"
 #include "kernels.hpp"
 #include "solver.hpp"
@@ -341,7 +342,7 @@ struct Physics final : PhysicsBase {
             upload(su, dst_basis<T>(g.Nom, g.Nmu, g.Nom));
             upload(sv, dst_basis<T>(g.Nmu, g.Nmu, g.Nom));
             if (std::is_same_v<T, float> &&
-                AnglePlanBuffers::usable(g.Nmu, g.Nom, static_cast<long long>(g.Ng) * nyz))
+                angle_on_matrix_cores(g.Nmu, g.Nom, static_cast<long long>(g.Ng) * nyz))
                 angle_plan.build(g.Nmu, g.Nom, s);
             if (secondary) {
                 for (int r = 0; r < g.Ng; ++r)
@@ -1514,8 +1515,9 @@ using namespace bfpn;
 // tables (stream-ordered, no host round trip).  Two operand sets are built on
 // the host and kept: the secondary source's operands (keyed by the kernel
 // table pointers and sizes; bfpn_secondary_source_prepare_* builds them) and
-// the CN factors of the angular step (keyed by the values of sig_tr and the
-// scalars).  A workspace orders its scratch on the stream of each call.
+// the CN factors and sine bases of the angular step (keyed by the kernel that
+// reads them, the values of sig_tr and the scalars).  A workspace orders its
+// scratch on the stream of each call.
 struct bfpn_workspace {
     struct SourceKey {
         const void *e1 = nullptr, *e2 = nullptr, *kv = nullptr, *beg = nullptr, *end = nullptr;
@@ -1531,7 +1533,7 @@ struct bfpn_workspace {
     AnglePlanBuffers angle_plan;
     SourceKey source_key;
     bool source_ready = false;
-    std::vector<double> angle_key;  // precision, grid scalars and sig_tr of the cached factors
+    std::vector<double> angle_key;  // angle_operand_key of the cached operands
     int builds = 0;                 // host-side builds of cached operands
 
     // Grows `b` to at least `bytes`.  Earlier calls on `s` may still read the
@@ -1651,10 +1653,9 @@ void op_angle(bfpn_workspace* ws, T* F, const double* sig_tr_host, int nyz, int 
     BFPN_REQUIRE(ws && F && sig_tr_host, "null argument");
     BFPN_REQUIRE(nyz > 0 && Ng > 0 && Nmu > 0 && Nom > 0 && Nmu * Nom <= 1024, "invalid sizes");
     const bool mfma = std::is_same_v<T, float> &&
-                      AnglePlanBuffers::usable(Nmu, Nom, static_cast<long long>(Ng) * nyz);
-    std::vector<double> key = {std::is_same_v<T, float> ? 0.0 : 1.0, double(Ng), double(Nmu),
-                               double(Nom), du, dv, dt, rho};
-    key.insert(key.end(), sig_tr_host, sig_tr_host + Ng);
+                      angle_on_matrix_cores(Nmu, Nom, static_cast<long long>(Ng) * nyz);
+    std::vector<double> key = angle_operand_key(std::is_same_v<T, double>, mfma, Ng, Nmu, Nom, du, dv,
+                                                dt, rho, sig_tr_host);
     if (key != ws->angle_key) {  // new tables: the buffers are rewritten after earlier calls
         BFPN_HIP(hipStreamSynchronize(s));
         ws->angle_key.clear();
