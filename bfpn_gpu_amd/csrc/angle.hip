@@ -419,15 +419,15 @@ __global__ __launch_bounds__(256) void angle_small_kernel(float* __restrict__ F_
 // 21 x 21 x 13 x 13 x 400 325 -> 235 us.
 constexpr int kRowThreads = 256;
 
-// y[j] = sum_k x[k] S[k][j], four sums at a time; done(j, y[j]) for each j.
+// y[j] = sum_k x[k] S[k][j], four sums at a time; done(j, y[j]) for each j < n.
 // S: blocked [j / 4][k][j % 4], 64 bytes per two k, requested two such chunks
 // ahead (the scheduling barrier keeps the request there; left to itself the
 // compiler loads all of S and spills scalar registers by the thousand).
 template <int N, typename Done>
-__device__ inline void dst_line(const double* __restrict__ S, const double (&x)[N], Done&& done) {
+__device__ inline void dst_line(const double* __restrict__ S, const double (&x)[N], int n, Done&& done) {
     typedef double f64x8 __attribute__((ext_vector_type(8)));
 #pragma unroll 1
-    for (int j = 0; j < N; j += 4) {
+    for (int j = 0; j < n; j += 4) {
         const f64x8* c = reinterpret_cast<const f64x8*>(S + j * N);
         f64x8 a = c[0], b = c[1];
         double acc[4] = {0.0, 0.0, 0.0, 0.0};
@@ -444,7 +444,8 @@ __device__ inline void dst_line(const double* __restrict__ S, const double (&x)[
             }
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) done(j + e, acc[e]);
+        for (int e = 0; e < 4; ++e)
+            if (j + e < n) done(j + e, acc[e]);
     }
 }
 
@@ -462,7 +463,8 @@ __global__ __launch_bounds__(kRowThreads) void angle_rows_kernel(
     const long long p0 = static_cast<long long>(blockIdx.x) * per_block;
     if (p0 >= active) return;
     // A plane holds NV rows of pitch values; the rows past Nmu and columns past
-    // Nom are zeros, and stay so: the padded bases make them.
+    // Nom are zeros and are never written (an infinity in the plane would make
+    // NaNs of them, and those spread to all of it).
     constexpr int pitch = NU | 1, plane = NV * pitch;
     double* X = reinterpret_cast<double*>(lds_raw);
     const int na = Nmu * Nom;
@@ -503,7 +505,7 @@ __global__ __launch_bounds__(kRowThreads) void angle_rows_kernel(
             double x[NU];
 #pragma unroll
             for (int a = 0; a < NU; ++a) x[a] = line[a];
-            dst_line<NU>(su, x, [&](int j, double y) { line[j] = y; });
+            dst_line<NU>(su, x, Nom, [&](int j, double y) { line[j] = y; });
         }
     };
     row_pass();  // Y[v][mu] = sum_a X[v][a] Su[mu][a]
@@ -519,10 +521,10 @@ __global__ __launch_bounds__(kRowThreads) void angle_rows_kernel(
         };
         // Z[nu][mu] = C[nu][mu] sum_v Sv[nu][v] Y[v][mu], in the column's place
         read();
-        dst_line<NV>(sv, x, [&](int j, double y) { line[j * pitch] = y * C[min(j, Nmu - 1) * Nom]; });
+        dst_line<NV>(sv, x, Nmu, [&](int j, double y) { line[j * pitch] = y * C[j * Nom]; });
         // W[v][mu] = sum_nu Sv[nu][v] Z[nu][mu]
         read();
-        dst_line<NV>(sv, x, [&](int j, double y) { line[j * pitch] = y; });
+        dst_line<NV>(sv, x, Nmu, [&](int j, double y) { line[j * pitch] = y; });
     }
     __syncthreads();
     row_pass();  // X'[v][a] = sum_mu W[v][mu] Su[mu][a]

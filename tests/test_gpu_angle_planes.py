@@ -75,3 +75,29 @@ def test_fp64_planes_against_the_oracle(gpu, oracle_mod, Nmu, Nom, nyz, Ng):
     gpu.ops.angle_full(d, sig, *args)
     err = np.abs(d.numpy().reshape(F.shape) - want.reshape(F.shape))
     assert np.all(err <= 1e-12 * np.abs(F).max(axis=(2, 3), keepdims=True))
+
+
+@pytest.mark.parametrize("Nmu,Nom", [(1, 1), (1, 2), (2, 1), (2, 2), (4, 6), (1, 12), (12, 1), (10, 4),
+                                     (22, 2), (30, 28)])
+@pytest.mark.parametrize("at", [(0, 0), (-1, -1)])
+def test_fp64_planes_with_an_infinity(gpu, oracle_mod, Nmu, Nom, at):
+    """The lines are padded, the sums are not: infinities and NaNs come out where
+    the plane's own values make them, and the other planes are untouched.  (Sizes
+    whose bases hold no zero: the sign of a rounded one would be arbitrary.)"""
+    nyz, Ng = 3, 2
+    rng = np.random.default_rng(10 * Nmu + Nom)
+    F = rng.standard_normal((Ng, nyz, Nmu, Nom))
+    F[1, 1][at] = np.inf
+    sig = rng.uniform(0.0, 4.0, Ng)
+    args = (nyz, Ng, Nmu, Nom, 0.2, 0.13, 0.05, 1.2)
+    want = F.ravel().copy()
+    with np.errstate(invalid="ignore"):
+        oracle_mod.angle_full(want, sig, *args)
+    d = gpu.DeviceArray(F)
+    gpu.ops.angle_full(d, sig, *args)
+    got = d.numpy().ravel()
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    ok = np.isfinite(want)
+    assert ok.sum() >= F.size - Nmu * Nom
+    assert np.abs(got[ok] - want[ok]).max() <= 1e-12 * np.abs(F[np.isfinite(F)]).max()
