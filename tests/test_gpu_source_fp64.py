@@ -30,3 +30,34 @@ def test_source_tiles(gpu, oracle_mod, Ng, nyz, nang):
     gpu.ops.secondary_source(*dev, *(gpu.DeviceArray(a) for a in (ke1, ke2, kv, beg, end)), Ng, nyz,
                              nang, 0.5)
     assert np.abs(dev[2].numpy() - want).max() <= 1e-12 * max(np.abs(want).max(), 1e-300)
+
+
+@pytest.mark.parametrize("low,high", [(24, 30), (32, 48), (19, 33), (47, 49)])
+def test_a_band_reads_its_own_groups_only(gpu, low, high):
+    """Output tiles of 16 groups with the same band [low, high) each, between
+    tiles whose bands are wider: infinite values in the source groups beside the
+    narrow band, and weights there that are no numbers, leave those tiles as
+    they are."""
+    Ng, nyz, nang = 80, 3, 5
+    rng = np.random.default_rng(low)
+    Fp, fp = rng.random((Ng, nyz * nang)), rng.standard_normal((Ng, nyz * nang))
+    kv = rng.random((Ng, nang, nang))
+    beg, end = np.full(Ng, 17, np.int32), np.full(Ng, 60, np.int32)
+    narrow = np.zeros(Ng, bool)
+    narrow[:16] = narrow[48:64] = True
+    beg[narrow], end[narrow] = low, high
+    inside = (np.arange(Ng) >= beg[:, None]) & (np.arange(Ng) < end[:, None])
+    ke1, ke2 = (np.where(inside, rng.random((Ng, Ng)), 0.0) for _ in range(2))
+    out = []
+    for spoil in (False, True):
+        X, e1, e2 = Fp.copy(), ke1.copy(), ke2.copy()
+        if spoil:
+            X[low - 1, 2] = X[high, 4] = np.inf
+            e1[~inside] = e2[~inside] = np.nan
+        dev = [gpu.DeviceArray(a.ravel()) for a in (X, fp, np.zeros((Ng, nyz * nang)))]
+        gpu.ops.secondary_source(*dev, *(gpu.DeviceArray(a) for a in (e1, e2, kv, beg, end)), Ng, nyz,
+                                 nang, 0.5)
+        out.append(dev[2].numpy().reshape(Ng, -1))
+    np.testing.assert_array_equal(out[1][narrow], out[0][narrow])
+    assert np.abs(out[0][narrow]).min() > 0.0
+    assert not np.isfinite(out[1][~narrow]).all()
