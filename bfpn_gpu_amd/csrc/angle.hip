@@ -667,9 +667,7 @@ void launch_angle_full(T* F, const T* factors, const T* su, const T* sv, int Ng,
             const long long blocks = (planes + per_block - 1) / per_block;
             BFPN_REQUIRE(blocks < (1LL << 31), "too many angular planes");
             auto go = [&](auto kernel) {
-                BFPN_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             static_cast<int>(lds)));
+                allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
                 hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kRowThreads),
                                    lds, s, F, factors, su, sv, planes, nyz, Nmu, Nom, per_block, top);
             };

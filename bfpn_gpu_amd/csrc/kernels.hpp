@@ -7,6 +7,12 @@
 
 namespace bfpn {
 
+// Lets `kernel` be launched with `bytes` of dynamic LDS (up to a CU's 160 KB).
+// The limit belongs to the kernel, not to a launch, and one kernel serves
+// several sizes: it is raised to the whole LDS once per kernel and device, so
+// no thread can lower it between another's request and launch.
+void allow_dynamic_lds(const void* kernel, size_t bytes);
+
 // Active energy groups.  Above the highest nonzero group ("top") of a beam
 // every group of the state is exactly zero: the energy sweep moves particles
 // down in energy (straggling spreads them at most one group up per half

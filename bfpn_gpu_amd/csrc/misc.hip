@@ -11,6 +11,11 @@
 
 #include "kernels.hpp"
 
+#include <algorithm>
+#include <mutex>
+#include <set>
+#include <utility>
+
 namespace bfpn {
 namespace {
 
@@ -316,6 +321,21 @@ void launch_yz_weights(int Ny, int Nz, bool trapezoidal, double* out, hipStream_
     hipLaunchKernelGGL(yz_weight_kernel, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, Ny, Nz,
                        trapezoidal ? 1 : 0, out);
     BFPN_HIP(hipGetLastError());
+}
+
+void allow_dynamic_lds(const void* kernel, size_t bytes) {
+    constexpr size_t kAlways = 64 * 1024, kWhole = 160 * 1024;  // every kernel's limit; a CU's LDS
+    BFPN_REQUIRE(bytes <= kWhole, "a work-group has at most 160 KB of LDS");
+    if (bytes <= kAlways) return;
+    static std::mutex mu;
+    static std::set<std::pair<int, const void*>> raised;
+    int dev = 0;
+    BFPN_HIP(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(mu);
+    if (raised.count({dev, kernel})) return;
+    BFPN_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 static_cast<int>(kWhole)));
+    raised.insert({dev, kernel});
 }
 
 // Groups per chunk of the dose kernel: about 1024 work-groups where the lanes

@@ -438,9 +438,7 @@ void launch_march(T* F, T* f, const T* omend, int Ny, int Nz, int Ng, int nang, 
     BFPN_REQUIRE(tiles < (1LL << 31) - 8, "transport grid too large");
     const dim3 grid(static_cast<unsigned>((tiles + 7) / 8 * 8), f ? 2 : 1);
     auto go = [&](auto kernel) {
-        BFPN_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     static_cast<int>(lds)));
+        allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
         hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, s, F, f, omend, Ny, Nz, nang,
                            static_cast<T>(1.0 / dy), static_cast<T>(1.0 / dz), static_cast<T>(h),
                            static_cast<int>(tiles), top);
