@@ -1432,18 +1432,38 @@ void validate_map(const std::vector<LayerSpec>& materials, const std::vector<dou
     for (unsigned char m : map) BFPN_REQUIRE(m < materials.size(), "map entry names no material");
 }
 
+static size_t elem_bytes(int precision) { return precision == BFPN_FP64 ? 8 : 4; }
+
+// Dose partials that admission counts for one closing energy sweep of a context:
+// one per 256 lanes, or its sweep's if those are more (its eb_).
+static size_t dose_partials(const bfpn_grid& g, const bfpn_phys& p, int precision) {
+    const long long lanes = static_cast<long long>(g.Ny + 1) * (g.Nz + 1) * g.Nmu * g.Nom;
+    const int least = upwind_blocks(lanes);
+    if (p.legacy_energy || p.lite_memory) return least;
+    return std::max(least, energy_blocks(lanes, g.Ng, elem_bytes(precision)));
+}
+
 size_t map_bytes(const bfpn_grid& g, const bfpn_phys& p, const std::vector<unsigned char>& map,
                  int nmat, int precision) {
     const size_t nyz = static_cast<size_t>(g.Ny + 1) * (g.Nz + 1);
+    const long long nang = static_cast<long long>(g.Nmu) * g.Nom;
     size_t minority = 0;  // the most nodes outside the largest material, over the slabs
+    const size_t plain = dose_partials(g, p, precision);
+    size_t partials = 2 * plain;  // the most dose and proxy partials of one sweep, likewise
     for (size_t j = 0; nyz && j + 1 <= map.size() / nyz; ++j) {
         std::vector<size_t> count(static_cast<size_t>(std::max(nmat, 1)), 0);
         for (size_t s = 0; s < nyz; ++s) ++count[std::min<size_t>(map[j * nyz + s], count.size() - 1)];
-        minority = std::max(minority, nyz - *std::max_element(count.begin(), count.end()));
+        const auto major = std::max_element(count.begin(), count.end());
+        minority = std::max(minority, nyz - *major);
+        size_t n = 0;
+        for (auto c = count.begin(); c != count.end(); ++c)
+            if (*c) n += 2 * energy_blocks((c == major ? nyz : *c) * nang, g.Ng, elem_bytes(precision));
+        partials = std::max(partials, n);
     }
     const bool sec = !p.primary_only && !p.energy_only && !p.lite_memory;
-    const size_t word = precision == BFPN_FP64 ? 8 : 4;
-    return (sec ? 8 : 2) * minority * g.Ng * g.Nmu * g.Nom * word;
+    const size_t word = elem_bytes(precision);
+    return (sec ? 8 : 2) * minority * g.Ng * g.Nmu * g.Nom * word +
+           (5 * partials - 9 * plain) * 8;  // in place of a plain context's
 }
 
 bfpn_ctx* make_mapped_context(const bfpn_grid& g, const bfpn_phys& p,
@@ -1488,9 +1508,9 @@ bfpn_ctx* make_mapped_context(const bfpn_grid& g, const bfpn_phys& p,
 size_t context_bytes(const bfpn_grid& g, const bfpn_phys& p, int precision) {
     const size_t lanes = static_cast<size_t>(g.Ny + 1) * (g.Nz + 1) * g.Nmu * g.Nom;
     const size_t cells = lanes * g.Ng;
-    const size_t word = precision == BFPN_FP64 ? 8 : 4;
+    const size_t word = elem_bytes(precision);
     const bool sec = !p.primary_only && !p.energy_only && !p.lite_memory;
-    return cells * word * (p.lite_memory ? 1 : sec ? 10 : 4) + 9 * ((lanes + 255) / 256) * 8 +
+    return cells * word * (p.lite_memory ? 1 : sec ? 10 : 4) + 9 * dose_partials(g, p, precision) * 8 +
            2 * static_cast<size_t>(std::max(16, g.Nx)) * 8;
 }
 
