@@ -47,6 +47,15 @@ constexpr int waves_per_simd() {
     return sizeof(T) == 4 ? (P == 1 ? 8 : P == 2 ? 5 : 4) : (P == 1 ? 4 : 3);
 }
 
+// Step t loads row t + this: the rows t + 3 .. are in flight.  Four wherever a
+// row is many cache lines: an XCD's work-groups hold that many rows of their
+// planes in its 4 MB L2, and with seven the lines that neighbouring chunks of
+// directions share were fetched twice (81 x 81 x 400 x 500 FP32 steps 203.4 ms
+// in a whole march, 198.7 with six, 197.2 with four).  Seven hides the latency
+// of short marches better where one column a thread leaves the lines few.
+template <typename T, int P>
+constexpr int rows_ahead() { return sizeof(T) == 4 && P == 1 ? 7 : 4; }
+
 // LDS slots of MW values per y column (two rows each of psi, psi* and their
 // y slopes), and the distance of
 // two columns: chosen so that the P columns a thread steps over amount to MW
@@ -104,17 +113,18 @@ __device__ inline T limited_slope(T a, T b) {
 // a slot is rewritten one barrier after its last reader.
 //
 // The z march is unrolled by 8: the psi window and the rows in flight share
-// one register ring indexed by row mod 8 (row t+7 is loaded into the slot of
-// row t-1, which step t no longer reads), so sliding a window is a renaming
+// one register ring indexed by row mod 8 (row t+4 or t+7 is loaded into a slot
+// that step t no longer reads), so sliding a window is a renaming
 // rather than a chain of moves and a loaded row is never copied (a copy would
 // wait for the load).  Rows past Nz are loaded as copies of row Nz: with them,
 // and with zero slopes carried into rows 0, the clamped stencil at both ends
 // needs no selects.  The first four steps (Start) and the last ones (End)
 // leave out the halves that have no row to work on; those tests are uniform.
 //
-// A corrector adds its two axes' terms in one order up to the step t with
-// t + 13 > Nz and at t = 2, 3 the other way round (Upper and beyond): a choice
-// without meaning that keeps results bit for bit what they have been.
+// A corrector adds its two axes' terms in one order in the blocks of eight steps
+// that start 13 or more rows before Nz and the other way round elsewhere (at
+// t = 2, 3, and from Upper on): a choice without meaning that keeps values what
+// they have been.
 //
 // What bounds it: vector issue and HBM together (47 vector instructions, 8
 // bytes per cell).  Against a march with four-row rings in LDS (12 LDS
@@ -145,7 +155,7 @@ __device__ __forceinline__ void transport_march(T* __restrict__ F, const T* __re
     if (L >= active) return;
     const int g = L / mchunks;
     T* ring = reinterpret_cast<T*>(lds_raw);
-    constexpr int YP = column_pitch<MW, P>();
+    constexpr int YP = column_pitch<MW, P>(), A = rows_ahead<T, P>();
     constexpr int kPsi = 0, kPred = 2, kS = 4, kSPred = 6;  // first slot of each ring
 
     // A thread whose columns would pass Ny takes the last P instead: the ones
@@ -176,7 +186,7 @@ __device__ __forceinline__ void transport_march(T* __restrict__ F, const T* __re
     unsigned soff[P];  // the same for stores; kOutside (dropped) for copies
     T* const own = ring + y0 * YP + mm;  // LDS: the thread's first column,
     const T *left, *right, *near[P];     // the ones beside it, the upwind ones (clamped)
-    T win[P][8];    // psi rows t .. t+2, then rows t+3 .. t+7 in flight (row mod 8)
+    T win[P][8];    // psi rows t .. t+2, then rows t+3 .. t+A in flight (row mod 8)
     T wpred[P][4];  // psi*, rows t-2 .. t after the predictor of step t (row mod 4)
     T wbase[P][4];  // psi - h/2 L(psi), the same rows
     T sy[P][2], dn[P][2];    // y slope and c - (upwind neighbour) of psi rows t, t+1
@@ -194,7 +204,7 @@ __device__ __forceinline__ void transport_march(T* __restrict__ F, const T* __re
             soff[j] = (y >= first && live) ? boff[j] : kOutside;
             near[j] = column(py ? y - 1 : y + 1);
 #pragma unroll
-            for (int r = 0; r < 7; ++r)
+            for (int r = 0; r < A; ++r)
                 win[j][r] = bload<T>(Fg, boff[j], static_cast<unsigned>(min(r, Nz)) * zbytes);
             sz[j] = szp[j] = uz[j] = uzp[j] = T(0);
         }
@@ -247,11 +257,10 @@ __device__ __forceinline__ void transport_march(T* __restrict__ F, const T* __re
         // Keep each step's arithmetic after its barrier: moved earlier, the z
         // differences of later rows would wait for rows still in flight.
         __builtin_amdgcn_sched_barrier(0);
-        // row t+7 into the register slot of row t-1: five rows in flight
-        if (S != Part::End) {
-            const unsigned so = static_cast<unsigned>(min(t + 7, Nz)) * zbytes;
+        if (S != Part::End) {  // row t + A into a free register slot
+            const unsigned so = static_cast<unsigned>(min(t + A, Nz)) * zbytes;
 #pragma unroll
-            for (int j = 0; j < P; ++j) win[j][(k8 + 7) & 7] = bload<T>(Fg, boff[j], so);
+            for (int j = 0; j < P; ++j) win[j][(k8 + A) & 7] = bload<T>(Fg, boff[j], so);
         }
         // LDS reads of the step, issued together
         T al = T(0), ar = T(0), bl = T(0), br = T(0), en[P], cn[P];
@@ -357,9 +366,9 @@ __device__ __forceinline__ void transport_march(T* __restrict__ F, const T* __re
         block(t0, I4{}, Upper{});
         block(t0 + 4, I0{}, Upper{});
     }
-    // at most 10 steps are left; rows up to Nz + 2 are loaded in the first three
+    // at most 10 steps are left, and rows up to Nz + 2 <= t0 + 9 to load
     block(t0, I4{}, EndLoad{});
-    block(t0 + 4, I0{}, End{});
+    block(t0 + 4, I0{}, std::conditional_t<(A < 6), EndLoad, End>{});
     step(t0 + 8, I4{}, End{});
     step(t0 + 9, std::integral_constant<int, 5>{}, End{});
 }
@@ -390,29 +399,42 @@ struct MarchShape {
     int MW, P, threads;
 };
 
-// Launch shape of a plane of Ny1 columns.
-// FP32: the first of (directions, columns per thread) = (16, 1), (16, 2),
-// (8, 2), (8, 3) whose work-group fits.  8 directions are 32-byte row segments
-// (254 against 195 us at 21 x 21 nodes x 400 directions x 500 groups), so they
-// are for the widest planes.  More columns per thread than needed share more
-// differences but leave fewer waves per SIMD: two cost 18.8 against 17.0 us at
-// 13 x 13 x 81 x 500 and the same over whole 21 x 21 beam steps; three at 81 x 81
-// were 2 % faster alone (1.35 ms, x 400 x 250) and slowed the whole step, where
-// the other stream's kernels run beside them, from 47.6 to 50.7 ms.
+// Launch shape of `Ng` planes of Ny1 columns and nang directions.
+//
+// FP32: 16 directions (64-byte row segments) and one column per thread up to 64
+// columns.  From there on to 96 columns 32 directions, whole cache lines, and
+// three columns: four steps of a whole march at 81 x 81 nodes x 400 directions x
+// 500 groups 197.2 ms against 198.9 with (16, 2); alone, 81 x 21 x 121 x 500 203
+// against 261 us, 65 x 41 x 400 x 300 572 against 685.  A CU holds one such
+// work-group, so where their last round would leave much of the chip idle (81 x
+// 81 x 400 x 60, 780 of them: 327 against 300 us; 81 x 81 x 81 x 120, 360: 144
+// against 113) the smaller ones of (16, 2) are kept.  More columns per thread
+// than needed share more differences but leave fewer waves per SIMD: two cost
+// 18.8 against 17.0 us at 13 x 13 x 81 x 500.  8 directions are 32-byte segments
+// (254 against 195 us at 21 x 21 x 400 x 500): for the widest planes.
+//
 // FP64: a thread's windows allow four waves per SIMD, so what counts is how
-// many of a CU's 16 wave slots whole work-groups fill: 24 directions (two
-// work-groups of 8 waves) at 21 columns, 198 us for 400 x 300, against 252 with
-// 16 (two of 6) and 206 with 8; 8 directions at 81 columns.  Wider planes take
-// several columns per thread.
-MarchShape march_shape(int Ny1, int nang, size_t elem) {
+// many work-groups that leaves per CU: 16 / waves up to four waves, beyond that
+// 4 / (waves on its fullest SIMD).  24 directions at 21 columns (two work-groups
+// of 8 waves), 158 us for 400 x 250, against 200 with 16 (two of 6) and 170 with
+// 8; but at 13 columns (two of 5 waves against four of 4) 162 against 128 us
+// x 500.  8 directions, half lines, need the other half's work-group near: up to
+// 28 columns, or 36 where a group has few chunks (31 x 31 x 81 x 500 195 against
+// 168 us with 16, but 49 directions 86 against 107), and 49 columns and more,
+// where 16 do not fit.  Their cost counts 6 % more.  Planes above 96 columns take
+// two columns per thread.
+MarchShape march_shape(int Ny1, int nang, int Ng, size_t elem) {
     auto threads_of = [&](int MW, int P) { return (MW * ((Ny1 + P - 1) / P) + 63) / 64 * 64; };
+    auto tiles_of = [&](int MW) { return static_cast<long long>((nang + MW - 1) / MW) * Ng; };
     MarchShape best{0, 0, 0};
     if (elem == 8) {
         double least = 0.0;
         for (const int MW : {16, 24, 8}) {
             const int threads = threads_of(MW, 1), waves = threads / 64;
             if (threads > max_threads<double>()) continue;
-            const double cost = static_cast<double>((nang + MW - 1) / MW) / (16 / waves);
+            if (MW == 8 && best.MW && Ny1 > (nang <= 64 ? 36 : 28)) continue;
+            const int resident = waves <= 4 ? 16 / waves : 4 / ((waves + 3) / 4);
+            const double cost = (MW == 8 ? 1.06 : 1.0) * ((nang + MW - 1) / MW) / resident;
             if (best.MW && cost >= least) continue;
             least = cost;
             best = MarchShape{MW, 1, threads};
@@ -420,9 +442,10 @@ MarchShape march_shape(int Ny1, int nang, size_t elem) {
         // (two columns per thread reach 192 columns; the limit is 170)
         return best.MW ? best : MarchShape{8, 2, threads_of(8, 2)};
     }
-    constexpr int cand[][2] = {{16, 1}, {16, 2}, {8, 2}, {8, 3}};
+    constexpr int cand[][2] = {{16, 1}, {32, 3}, {16, 2}, {8, 2}, {8, 3}};
     for (const auto& c : cand) {
         const int MW = c[0], P = c[1], threads = threads_of(MW, P);
+        if (MW == 32 && tiles_of(MW) * 5 < (tiles_of(MW) + 255) / 256 * 256 * 4) continue;  // 256 CUs, 80 %
         if (threads <= max_threads<float>()) return MarchShape{MW, P, threads};
     }
     return best;
@@ -468,7 +491,7 @@ void launch_transport_half(T* F, const T* omend, int Ny, int Nz, int Ng, int nan
     // one group's block is addressed with 32-bit byte offsets
     BFPN_REQUIRE(static_cast<long long>(Ny + 1) * (Nz + 1) * nang * sizeof(T) < (1LL << 31),
                  "transport needs (Ny+1)(Nz+1)*Nmu*Nom values of one energy group below 2 GiB");
-    const MarchShape sh = march_shape(Ny + 1, nang, sizeof(T));
+    const MarchShape sh = march_shape(Ny + 1, nang, Ng, sizeof(T));
 #define BFPN_MARCH(MW_, P_)                                                                   \
     if (sh.MW == MW_ && sh.P == P_)                                                           \
         return launch_march<T, MW_, P_>(F, f, omend, Ny, Nz, Ng, nang, sh.threads, dy, dz, h,     \
@@ -476,6 +499,7 @@ void launch_transport_half(T* F, const T* omend, int Ny, int Nz, int Ng, int nan
     BFPN_MARCH(16, 1);
     BFPN_MARCH(8, 2);
     if constexpr (sizeof(T) == 4) {
+        BFPN_MARCH(32, 3);
         BFPN_MARCH(16, 2);
         BFPN_MARCH(8, 3);
     } else {
