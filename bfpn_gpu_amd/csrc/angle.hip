@@ -419,15 +419,15 @@ __global__ __launch_bounds__(256) void angle_small_kernel(float* __restrict__ F_
 // 21 x 21 x 13 x 13 x 400 325 -> 235 us.
 constexpr int kRowThreads = 256;
 
-// y[j] = sum_k x[k] S[k][j], four sums at a time; done(j, y[j]) for each j < n.
+// y[j] = sum_k x[k] S[k][j], four sums at a time; done(j, y[j]) for each j.
 // S: blocked [j / 4][k][j % 4], 64 bytes per two k, requested two such chunks
 // ahead (the scheduling barrier keeps the request there; left to itself the
 // compiler loads all of S and spills scalar registers by the thousand).
 template <int N, typename Done>
-__device__ inline void dst_line(const double* __restrict__ S, const double (&x)[N], int n, Done&& done) {
+__device__ inline void dst_line(const double* __restrict__ S, const double (&x)[N], Done&& done) {
     typedef double f64x8 __attribute__((ext_vector_type(8)));
 #pragma unroll 1
-    for (int j = 0; j < n; j += 4) {
+    for (int j = 0; j < N; j += 4) {
         const f64x8* c = reinterpret_cast<const f64x8*>(S + j * N);
         f64x8 a = c[0], b = c[1];
         double acc[4] = {0.0, 0.0, 0.0, 0.0};
@@ -444,14 +444,13 @@ __device__ inline void dst_line(const double* __restrict__ S, const double (&x)[
             }
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (j + e < n) done(j + e, acc[e]);
+        for (int e = 0; e < 4; ++e) done(j + e, acc[e]);
     }
 }
 
 // su, sv: the bases padded to NU x NU and NV x NV, blocked as dst_line reads
-// them.
-template <int NU, int NV>
+// them.  EXACT: the plane is NV x NU and nothing is padded.
+template <int NU, int NV, bool EXACT>
 __global__ __launch_bounds__(kRowThreads) void angle_rows_kernel(
     double* __restrict__ F, const double* __restrict__ factors, const double* __restrict__ su,
     const double* __restrict__ sv, long long planes, int nyz, int Nmu, int Nom, int per_block,
@@ -462,19 +461,17 @@ __global__ __launch_bounds__(kRowThreads) void angle_rows_kernel(
             : planes;
     const long long p0 = static_cast<long long>(blockIdx.x) * per_block;
     if (p0 >= active) return;
-    // A plane holds NV rows of pitch values; the rows past Nmu and columns past
-    // Nom are zeros and are never written (an infinity in the plane would make
-    // NaNs of them, and those spread to all of it).
+    // A plane holds NV rows of pitch values, at most three rows past Nmu and
+    // columns past Nom.  Those are read as zeros whatever they hold: the padded
+    // bases make NaNs of them where the plane holds an infinity, which would
+    // spread to all of it.  (Kept out at the stores instead, by a select 3 %, by
+    // a branch, which spills scalar registers, up to four times as slow.)
     constexpr int pitch = NU | 1, plane = NV * pitch;
     double* X = reinterpret_cast<double*>(lds_raw);
     const int na = Nmu * Nom;
     const int np = static_cast<int>(min(static_cast<long long>(per_block), active - p0));
     const int rows = np * Nmu, cols = np * Nom, n = np * na;
     double* base = F + p0 * na;
-    if (Nmu < NV || Nom < NU) {
-        for (int e = threadIdx.x; e < np * plane; e += kRowThreads) X[e] = 0.0;
-        __syncthreads();
-    }
     // coalesced copy of the run: value e sits at column c of row v of a plane;
     // a step of kRowThreads values is dp planes, dv rows and dc columns
     const int dr = kRowThreads / Nom, dc = kRowThreads - dr * Nom, dp = dr / Nmu, dv = dr - dp * Nmu;
@@ -504,8 +501,8 @@ __global__ __launch_bounds__(kRowThreads) void angle_rows_kernel(
             double* line = X + p * plane + (r - p * Nmu) * pitch;
             double x[NU];
 #pragma unroll
-            for (int a = 0; a < NU; ++a) x[a] = line[a];
-            dst_line<NU>(su, x, Nom, [&](int j, double y) { line[j] = y; });
+            for (int a = 0; a < NU; ++a) x[a] = EXACT || a < NU - 3 || a < Nom ? line[a] : 0.0;
+            dst_line<NU>(su, x, [&](int j, double y) { line[j] = y; });
         }
     };
     row_pass();  // Y[v][mu] = sum_a X[v][a] Su[mu][a]
@@ -517,14 +514,14 @@ __global__ __launch_bounds__(kRowThreads) void angle_rows_kernel(
         double x[NV];
         auto read = [&] {
 #pragma unroll
-            for (int v = 0; v < NV; ++v) x[v] = line[v * pitch];
+            for (int v = 0; v < NV; ++v) x[v] = EXACT || v < NV - 3 || v < Nmu ? line[v * pitch] : 0.0;
         };
         // Z[nu][mu] = C[nu][mu] sum_v Sv[nu][v] Y[v][mu], in the column's place
         read();
-        dst_line<NV>(sv, x, Nmu, [&](int j, double y) { line[j * pitch] = y * C[j * Nom]; });
+        dst_line<NV>(sv, x, [&](int j, double y) { line[j * pitch] = y * C[min(j, Nmu - 1) * Nom]; });
         // W[v][mu] = sum_nu Sv[nu][v] Z[nu][mu]
         read();
-        dst_line<NV>(sv, x, Nmu, [&](int j, double y) { line[j * pitch] = y; });
+        dst_line<NV>(sv, x, [&](int j, double y) { line[j * pitch] = y; });
     }
     __syncthreads();
     row_pass();  // X'[v][a] = sum_mu W[v][mu] Su[mu][a]
@@ -673,19 +670,32 @@ void launch_angle_full(T* F, const T* factors, const T* su, const T* sv, int Ng,
             };
             auto with_nu = [&](auto u) {
                 constexpr int NU = decltype(u)::value;
+                auto with_nv = [&](auto v) {
+                    constexpr int NV = decltype(v)::value;
+                    if (Nom == NU && Nmu == NV)
+                        go(&angle_rows_kernel<NU, NV, true>);
+                    else
+                        go(&angle_rows_kernel<NU, NV, false>);
+                };
                 switch (nv) {
-                    case 8: go(&angle_rows_kernel<NU, 8>); break;
-                    case 12: go(&angle_rows_kernel<NU, 12>); break;
-                    case 16: go(&angle_rows_kernel<NU, 16>); break;
-                    case 20: go(&angle_rows_kernel<NU, 20>); break;
-                    default: go(&angle_rows_kernel<NU, 32>); break;
+                    case 4: with_nv(std::integral_constant<int, 4>{}); break;
+                    case 8: with_nv(std::integral_constant<int, 8>{}); break;
+                    case 12: with_nv(std::integral_constant<int, 12>{}); break;
+                    case 16: with_nv(std::integral_constant<int, 16>{}); break;
+                    case 20: with_nv(std::integral_constant<int, 20>{}); break;
+                    case 24: with_nv(std::integral_constant<int, 24>{}); break;
+                    case 28: with_nv(std::integral_constant<int, 28>{}); break;
+                    default: with_nv(std::integral_constant<int, 32>{}); break;
                 }
             };
             switch (nu) {
+                case 4: with_nu(std::integral_constant<int, 4>{}); break;
                 case 8: with_nu(std::integral_constant<int, 8>{}); break;
                 case 12: with_nu(std::integral_constant<int, 12>{}); break;
                 case 16: with_nu(std::integral_constant<int, 16>{}); break;
                 case 20: with_nu(std::integral_constant<int, 20>{}); break;
+                case 24: with_nu(std::integral_constant<int, 24>{}); break;
+                case 28: with_nu(std::integral_constant<int, 28>{}); break;
                 default: with_nu(std::integral_constant<int, 32>{}); break;
             }
             BFPN_HIP(hipGetLastError());

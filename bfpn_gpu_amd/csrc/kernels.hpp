@@ -157,7 +157,7 @@ void launch_transport_half(T* F, const T* omend, int Ny, int Nz, int Ng, int nan
 // su, sv: the sine bases of Nom and Nmu (T), Nom*Nom and Nmu*Nmu, or, FP64 up to
 // 32 x 32 directions, each padded with zeros to np = dst_pitch() rows and columns
 // and blocked: entry (k, j) at [j / 4][k][j % 4].
-constexpr int dst_pitch(int n) { return n <= 8 ? 8 : n <= 20 ? (n + 3) / 4 * 4 : 32; }
+constexpr int dst_pitch(int n) { return (n + 3) / 4 * 4; }
 template <typename T>
 void launch_angle_full(T* F, const T* factors, const T* su, const T* sv, int Ng, int nyz, int Nmu,
                        int Nom, hipStream_t s, const int* top = nullptr);
