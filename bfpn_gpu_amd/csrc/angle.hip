@@ -11,9 +11,11 @@
 // runs per (g, s) plane of Nmu x Nom values, in place.  The CN factors
 // (ratio * DST normalisation) are built once on the host per (g, direction).
 // FP32 state: matrix cores, stages chained in registers (below).  FP64 state:
-// vector kernel, a thread per row or column of a plane.  Planes wider than 32:
-// vector kernel with the plane and bases in LDS.
+// vector kernel, a thread per row or column of a plane.  Planes wider than 32,
+// and thin ones in FP64 (angle_by_lines): vector kernel, a thread per value,
+// with the plane and bases in LDS.
 
+#include "angle_operands.hpp"
 #include "buffer.hpp"
 #include "kernels.hpp"
 #include "mfma.hpp"
@@ -402,7 +404,7 @@ __global__ __launch_bounds__(256) void angle_small_kernel(float* __restrict__ F_
 }
 
 // ------------------------------------------------------- FP64, vector ------
-// FP64 planes of at most 32 x 32: one thread per row, then per column, then per
+// FP64 planes of at most 32 x 32, not thin: one thread per row, then per column, then per
 // row of a plane, its line in registers, the bases through the scalar cache
 // (they are uniform, so a multiply-add reads its basis value from an SGPR and
 // needs one operand of the line).  The column pass does both inner stages and
@@ -655,8 +657,8 @@ void launch_angle_full(T* F, const T* factors, const T* su, const T* sv, int Ng,
     const long long planes = static_cast<long long>(Ng) * nyz;
     if (planes == 0) return;
     if constexpr (sizeof(T) == 8) {
-        const int widest = std::max(Nmu, Nom);
-        if (widest <= 32) {
+        if (angle_by_lines(Nmu, Nom)) {
+            const int widest = std::max(Nmu, Nom);
             const int nu = dst_pitch(Nom), nv = dst_pitch(Nmu);
             // one line per thread in the passes over the longer axis
             const int per_block = std::max(1, kRowThreads / widest);

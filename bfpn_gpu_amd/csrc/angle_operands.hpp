@@ -2,6 +2,7 @@
 // operands (standard C++ only).
 #pragma once
 
+#include <algorithm>
 #include <vector>
 
 namespace bfpn {
@@ -11,6 +12,19 @@ namespace bfpn {
 // (launch_angle_mfma); other grids take the vector kernel.
 inline bool angle_on_matrix_cores(int Nmu, int Nom, long long planes) {
     return Nmu <= 32 && Nom <= 32 && planes < (1LL << 30) && planes * Nmu * Nom < (1LL << 31);
+}
+
+// Whether FP64 planes run a line per thread (bases padded and blocked) or a value
+// per thread.  Lines are the faster from 3 directions on (8 x 2 24 against 35 us,
+// 21 x 21 nodes x 500 groups), but thin planes are mostly their padding to four:
+// 1 x 20 directions 94 against 68 us, 27 x 2 211 against 142, 29 x 3 293 against
+// 232.  Not where the value kernel's LDS columns fall on few banks: 1 x 16 56
+// against 122 us, 2 x 24 142 against 302, 1 x 32 241 against 441.
+inline bool angle_by_lines(int Nmu, int Nom) {
+    const int least = std::min(Nmu, Nom), most = std::max(Nmu, Nom);
+    const bool few_banks = most % 8 == 0 && most > 8;
+    const bool thin = (least <= 2 && most > 4 * least) || (Nom == 3 && Nmu > 24);
+    return most <= 32 && (!thin || few_banks);
 }
 
 // Everything the operands of one call are built from.  The kernel belongs to

@@ -154,8 +154,8 @@ void launch_transport_half(T* F, const T* omend, int Ny, int Nz, int Ng, int nan
                            const int* top = nullptr, T* f = nullptr);
 
 // CN angular diffusion on the DST-I basis, in place.  factors: Ng*nang (T);
-// su, sv: the sine bases of Nom and Nmu (T), Nom*Nom and Nmu*Nmu, or, FP64 up to
-// 32 x 32 directions, each padded with zeros to np = dst_pitch() rows and columns
+// su, sv: the sine bases of Nom and Nmu (T), Nom*Nom and Nmu*Nmu, or, FP64 planes
+// of angle_by_lines(), each padded with zeros to np = dst_pitch() rows and columns
 // and blocked: entry (k, j) at [j / 4][k][j % 4].
 constexpr int dst_pitch(int n) { return (n + 3) / 4 * 4; }
 template <typename T>

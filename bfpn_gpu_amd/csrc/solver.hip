@@ -253,7 +253,7 @@ namespace {
 template <typename T>
 std::vector<T> dst_basis(int n, int Nmu, int Nom) {
     const auto s = sine_basis(n);
-    if (sizeof(T) == 4 || std::max(Nmu, Nom) > 32) return cast_vector<T>(s);
+    if (sizeof(T) == 4 || !angle_by_lines(Nmu, Nom)) return cast_vector<T>(s);
     const int np = dst_pitch(n);
     std::vector<T> pad(static_cast<size_t>(np) * np, T(0));
     for (int r = 0; r < n; ++r)

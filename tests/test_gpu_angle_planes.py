@@ -101,3 +101,22 @@ def test_fp64_planes_with_an_infinity(gpu, oracle_mod, Nmu, Nom, at):
     ok = np.isfinite(want)
     assert ok.sum() >= F.size - Nmu * Nom
     assert np.abs(got[ok] - want[ok]).max() <= 1e-12 * np.abs(F[np.isfinite(F)]).max()
+
+
+@pytest.mark.parametrize("Nmu,Nom", [(1, 4), (1, 5), (5, 1), (1, 8), (1, 16), (17, 1), (2, 8), (2, 9),
+                                     (9, 2), (2, 16), (24, 2), (24, 3), (25, 3), (3, 25), (31, 3),
+                                     (32, 3), (4, 29), (23, 24), (28, 27)])
+def test_fp64_thin_planes_and_every_padding(gpu, oracle_mod, Nmu, Nom):
+    """Both sides of the line between a thread per line and a thread per value,
+    exact and padded lines; the bound of the planes above."""
+    nyz, Ng = 37, 3
+    rng = np.random.default_rng(100 * Nmu + Nom)
+    F = rng.standard_normal((Ng, nyz, Nmu, Nom))
+    sig = rng.uniform(0.0, 4.0, Ng)
+    args = (nyz, Ng, Nmu, Nom, 0.2, 0.13, 0.05, 1.2)
+    want = F.ravel().copy()
+    oracle_mod.angle_full(want, sig, *args)
+    d = gpu.DeviceArray(F)
+    gpu.ops.angle_full(d, sig, *args)
+    err = np.abs(d.numpy().reshape(F.shape) - want.reshape(F.shape))
+    assert np.all(err <= 1e-12 * np.abs(F).max(axis=(2, 3), keepdims=True))
