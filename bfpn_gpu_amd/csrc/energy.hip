@@ -512,15 +512,24 @@ constexpr int kSplitRing = 16;  // groups per LDS chunk, the unroll
 template <typename T, bool FOUR>
 constexpr int split_ring() { return FOUR || sizeof(T) == 8 ? 8 : 16; }
 
-// Lanes of one array from which one thread per lane is the better sweep: 2^16
-// lanes are 2048 waves here, the two per SIMD that its registers allow; one
-// more round of waves costs what the split gains.  Measured (FP32, straggling,
-// primary with its copy and secondary with two sources, mean of the two, one
-// kernel at a time): 14,641 lanes x 500 groups 207 -> 83 us, 25,600 x 500
-// 207 -> 105 us, 46,656 x 400 176 -> 104 us; 74,529 x 400 214 -> 243 us.
-constexpr long long kSplitLanes = 1LL << 16;
-inline bool energy_split(long long lanes, int Ng, size_t elem) {
-    return lanes < kSplitLanes && lanes * Ng * static_cast<long long>(elem) < (1LL << 31);
+// Lanes of one array from which one thread per lane is the better sweep.  32,768
+// lanes are one wave here for every SIMD; beyond that some SIMDs run two, which a
+// paired sweep's registers allow in FP32 only, and one thread per lane starts to
+// fill the chip.  Sweeps with dose sums, most of them paired (eight steps of a
+// march x 250 groups, split against not): FP32 38,416 lanes 2.35 against 2.52 ms,
+// 43,264 2.55 against 2.76, 44,100 2.84 against 2.82, 56,644 3.80 against 3.31;
+// FP64 23,716 4.68 against 5.02, 28,561 5.51 against 5.56, 33,124 6.33 against
+// 6.08, 56,644 11.2 against 10.2.  A single sweep without them has the registers
+// for two waves (one sweep x 250 groups): FP32 44,100 lanes 66 against 72 us,
+// 48,841 76 against 73, but where every row starts on a 64-byte boundary 50,176
+// 48 against 72 and 63,504 68 against 76; FP64 43,264 83 against 92, 44,100 107
+// against 100, 50,176 109 against 97.
+inline bool energy_split(long long lanes, int Ng, size_t elem, bool sums = true) {
+    const long long limit = sums ? (elem == 4 ? 44000 : 30000)
+                            : elem == 8      ? 43500
+                            : lanes % 16 == 0 ? (1LL << 16)
+                                              : 47000;
+    return lanes < limit && lanes * Ng * static_cast<long long>(elem) < (1LL << 31);
 }
 
 __device__ inline double swap_pair(double v) {
@@ -869,8 +878,8 @@ template <typename T, bool SRC, bool STRAG>
 void dispatch_lpt(T* F, T* f, const EnergyCoef* coef, const T* Q1, int Ng, long long lanes,
                   const double* yzw, int nang, double* partials, bool proxy, hipStream_t s,
                   const SweepTops& tops) {
-    if (energy_split(lanes, Ng, sizeof(T))) {
-        const dim3 grid(energy_blocks(lanes, Ng, sizeof(T)));
+    if (energy_split(lanes, Ng, sizeof(T), partials != nullptr)) {
+        const dim3 grid(static_cast<unsigned>((lanes + 31) / 32));
         T* const none = nullptr;
         if (partials)
             hipLaunchKernelGGL((energy_split_kernel<T, false, SRC, STRAG, true, false>), grid,

@@ -80,3 +80,44 @@ def test_both_arrays_in_one_launch(gpu, oracle_mod, over, no_clip):
             for k in range(4):
                 a, r = s.state(k), ref.state(k)
                 assert np.abs(a - r).max() <= tol * max(np.abs(r).max(), 1e-300)
+
+
+@pytest.mark.parametrize("dtype,lanes", [(np.float32, 46999), (np.float32, 47001), (np.float32, 47008),
+                                         (np.float32, 65520), (np.float32, 65536),
+                                         (np.float64, 43499), (np.float64, 43500)])
+def test_half_sweep_on_both_sides_of_its_limits(gpu, dtype, lanes):
+    """The split sweep and the one of a thread per lane: the same bits as the
+    first columns of a wide grid have."""
+    rng = np.random.default_rng(lanes)
+    Ng, wide = 19, (1 << 16) + 32
+    S, sig, T = 5.0 + 100.0 * rng.random(Ng + 1), 0.02 * rng.random(Ng), 0.01 * rng.random(Ng)
+    F, f, Q = (rng.standard_normal((Ng, wide)).astype(dtype) for _ in range(3))
+    tabs = [gpu.DeviceArray(a) for a in (S, sig, T)]
+
+    def run(cols):
+        a, b, q = (gpu.DeviceArray(np.ascontiguousarray(x[:, :cols])) for x in (F, f, Q))
+        gpu.ops.energy_half(a, b, *tabs, 0.01, 0.518, 1.1, Ng, cols, 1, Q1=q, straggling=True)
+        return a.numpy()[:, :lanes], b.numpy()[:, :lanes]
+
+    for narrow, full in zip(run(lanes), run(wide)):
+        np.testing.assert_array_equal(narrow, full)
+
+
+@pytest.mark.parametrize("precision,over", [("FP32", dict(Ny=12, Nz=15, Nmu=13, Nom=16)),   # 43,264
+                                            ("FP32", dict(Ny=13, Nz=14, Nmu=14, Nom=15)),   # 44,100
+                                            ("FP64", dict(Ny=8, Nz=16, Nmu=14, Nom=14)),    # 29,988
+                                            ("FP64", dict(Ny=10, Nz=13, Nmu=14, Nom=14))])  # 30,184
+def test_paired_sweep_on_both_sides_of_its_limits(gpu, oracle_mod, precision, over):
+    c = small_case(Ng=17, Lg=0.518 * 17, energy=5.0, flags=dict(eq15_straggling=1), **over)
+    ref = oracle_mod.Solver(c)
+    ref.advance(3)
+    tol = 1e-10 if precision == "FP64" else 2e-4
+    with gpu.Solver(c, getattr(gpu, precision)) as one, gpu.Solver(c, getattr(gpu, precision)) as many:
+        one.advance(3)
+        for _ in range(3):
+            many.advance(1)
+        np.testing.assert_allclose(one.history()[0], ref.history()[0], rtol=tol)
+        for k in range(4):
+            a, r = one.state(k), ref.state(k)
+            np.testing.assert_array_equal(a, many.state(k))
+            assert np.abs(a - r).max() <= tol * max(np.abs(r).max(), 1e-300)
