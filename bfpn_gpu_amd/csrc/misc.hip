@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <mutex>
 #include <set>
+#include <type_traits>
 #include <utility>
 
 namespace bfpn {
@@ -37,9 +38,14 @@ __device__ inline double block_sum256(double v, double* lds) {
 // thread walking all groups one at a time left a few waves waiting on each
 // load (21 x 21 nodes x 121 directions x 500 groups, four FP32 arrays, 427 MB:
 // 618 us = 0.69 TB/s, now 85 us = 5.0 TB/s).  HAS: bit 0 f, 1 F1, 2 f1 present.
+// WIDE (FP64 from kDoseWide lanes, where a walk of all groups with one load per
+// array in flight had enough threads already): six groups, non-temporal, for
+// arrays that no cache holds: 33 x 33 nodes x 400 directions x 120 groups 295 us
+// by that walk, 309 with eight groups and temporal loads, 276 so.
 constexpr int kDoseUnroll = 8;
+constexpr long long kDoseWide = 1LL << 17;
 
-template <typename T, int HAS>
+template <typename T, int HAS, bool WIDE>
 __global__ __launch_bounds__(kBlock) void dose_kernel(const T* __restrict__ F,
                                                       const T* __restrict__ f,
                                                       const T* __restrict__ F1,
@@ -48,7 +54,8 @@ __global__ __launch_bounds__(kBlock) void dose_kernel(const T* __restrict__ F,
                                                       const double* __restrict__ yzw, int Ng,
                                                       int chunk, long long lanes, int nang,
                                                       double* __restrict__ partials) {
-    constexpr int U = kDoseUnroll;
+    constexpr int U = WIDE ? 6 : kDoseUnroll;
+    auto at = [](const T* p) { return WIDE ? __builtin_nontemporal_load(p) : *p; };
     __shared__ double lds[kBlock / 64];
     const long long lane = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
     const int g0 = blockIdx.y * chunk, g1 = min(Ng, g0 + chunk);
@@ -66,18 +73,18 @@ __global__ __launch_bounds__(kBlock) void dose_kernel(const T* __restrict__ F,
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const long long idx = static_cast<long long>(g + u) * lanes + lane;
-                a[u] = F[idx];
-                b[u] = HAS & 1 ? f[idx] : T(0);
-                c[u] = HAS & 2 ? F1[idx] : T(0);
-                d[u] = HAS & 4 ? f1[idx] : T(0);
+                a[u] = at(F + idx);
+                b[u] = HAS & 1 ? at(f + idx) : T(0);
+                c[u] = HAS & 2 ? at(F1 + idx) : T(0);
+                d[u] = HAS & 4 ? at(f1 + idx) : T(0);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) add(g + u, a[u], b[u], c[u], d[u]);
         }
         for (; g < g1; ++g) {
             const long long idx = static_cast<long long>(g) * lanes + lane;
-            add(g, F[idx], HAS & 1 ? f[idx] : T(0), HAS & 2 ? F1[idx] : T(0),
-                HAS & 4 ? f1[idx] : T(0));
+            add(g, at(F + idx), HAS & 1 ? at(f + idx) : T(0), HAS & 2 ? at(F1 + idx) : T(0),
+                HAS & 4 ? at(f1 + idx) : T(0));
         }
         acc *= yzw[lane / nang];
     }
@@ -343,7 +350,7 @@ void allow_dynamic_lds(const void* kernel, size_t bytes) {
 // (512 and more) suffice, and the partial sums stay at one per lane block, which
 // is what the allocation-free dose's fixed scratch is sized for.
 static int dose_chunk(int Ng, long long lanes) {
-    if (lanes >= (1LL << 17) || Ng > (1 << 14)) return Ng;
+    if (lanes >= kDoseWide || Ng > (1 << 14)) return Ng;
     const int blocks = static_cast<int>((lanes + kBlock - 1) / kBlock);
     const int chunks = std::min((Ng + 2 * kDoseUnroll - 1) / (2 * kDoseUnroll), (1024 + blocks - 1) / blocks);
     const int per = (Ng + chunks - 1) / chunks;
@@ -367,15 +374,26 @@ void launch_dose(const T* F, const T* f, const T* F1, const T* f1, const DoseCoe
         hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, s, F, f, F1, f1, w, yz_weight, Ng, chunk,
                            lanes, nang, partials);
     };
-    switch (has) {
-        case 0: go(&dose_kernel<T, 0>); break;
-        case 1: go(&dose_kernel<T, 1>); break;
-        case 2: go(&dose_kernel<T, 2>); break;
-        case 3: go(&dose_kernel<T, 3>); break;
-        case 4: go(&dose_kernel<T, 4>); break;
-        case 5: go(&dose_kernel<T, 5>); break;
-        case 6: go(&dose_kernel<T, 6>); break;
-        default: go(&dose_kernel<T, 7>); break;
+    auto with = [&](auto wide) {
+        constexpr bool W = decltype(wide)::value;
+        switch (has) {
+            case 0: go(&dose_kernel<T, 0, W>); break;
+            case 1: go(&dose_kernel<T, 1, W>); break;
+            case 2: go(&dose_kernel<T, 2, W>); break;
+            case 3: go(&dose_kernel<T, 3, W>); break;
+            case 4: go(&dose_kernel<T, 4, W>); break;
+            case 5: go(&dose_kernel<T, 5, W>); break;
+            case 6: go(&dose_kernel<T, 6, W>); break;
+            default: go(&dose_kernel<T, 7, W>); break;
+        }
+    };
+    if constexpr (sizeof(T) == 8) {
+        if (lanes >= kDoseWide)
+            with(std::true_type{});
+        else
+            with(std::false_type{});
+    } else {
+        with(std::false_type{});
     }
     BFPN_HIP(hipGetLastError());
 }

@@ -35,6 +35,14 @@ def test_dose_over_chunks(gpu, oracle_mod, dtype, have, Ng, Ny, Nz, nang):
     assert abs(got - want) <= TOL * size
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("have", [0, 5, 7])
+@pytest.mark.parametrize("Ng,nang", [(5, 256), (6, 256), (7, 256), (7, 255)])
+def test_dose_of_wide_arrays(gpu, oracle_mod, dtype, have, Ng, nang):
+    """512 nodes: 2^17 lanes, and one direction fewer."""
+    test_dose_over_chunks(gpu, oracle_mod, dtype, have, Ng, 15, 31, nang)
+
+
 @pytest.mark.parametrize("Ng,over", [(2, dict(Ny=1, Nz=1, Nmu=1, Nom=1)),
                                      (17, dict(Ny=2, Nz=3, Nmu=7, Nom=9)),
                                      (65, dict(Ny=4, Nz=2, Nmu=8, Nom=9))])
