@@ -120,3 +120,23 @@ def test_fp64_thin_planes_and_every_padding(gpu, oracle_mod, Nmu, Nom):
     gpu.ops.angle_full(d, sig, *args)
     err = np.abs(d.numpy().reshape(F.shape) - want.reshape(F.shape))
     assert np.all(err <= 1e-12 * np.abs(F).max(axis=(2, 3), keepdims=True))
+
+
+@pytest.mark.parametrize("Nmu,Nom", [(1, 1), (3, 3), (5, 5), (8, 8), (7, 16), (16, 7), (12, 6), (11, 11),
+                                     (16, 16), (20, 20)])
+def test_a_plane_has_the_same_bits_wherever_it_sits(gpu, Nmu, Nom):
+    """Alone in a tile, and at every place of a tile that it shares with planes of
+    its own and of the next energy group."""
+    nyz, Ng = 5, 6
+    rng = np.random.default_rng(Nmu + 50 * Nom)
+    F = (rng.standard_normal((Ng, nyz, Nmu, Nom)) * 10.0 ** rng.uniform(-6, 6, (Ng, nyz, 1, 1)))
+    F = F.astype(np.float32)
+    sig = rng.uniform(0.0, 4.0, Ng)
+    d = gpu.DeviceArray(F)
+    gpu.ops.angle_full(d, sig, nyz, Ng, Nmu, Nom, 0.2, 0.13, 0.05, 1.2)
+    together = d.numpy().reshape(F.shape)
+    for g in range(Ng):
+        for s in range(nyz):
+            one = gpu.DeviceArray(np.ascontiguousarray(F[g, s]))
+            gpu.ops.angle_full(one, sig[g:g + 1], 1, 1, Nmu, Nom, 0.2, 0.13, 0.05, 1.2)
+            np.testing.assert_array_equal(one.numpy().reshape(Nmu, Nom), together[g, s])
