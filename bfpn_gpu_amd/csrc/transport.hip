@@ -47,12 +47,13 @@ constexpr int waves_per_simd() {
     return sizeof(T) == 4 ? (P == 1 ? 8 : P == 2 ? 5 : 4) : (P == 1 ? 4 : 3);
 }
 
-// Step t loads row t + this: the rows t + 3 .. are in flight.  Four wherever a
-// row is many cache lines: an XCD's work-groups hold that many rows of their
-// planes in its 4 MB L2, and with seven the lines that neighbouring chunks of
-// directions share were fetched twice (81 x 81 x 400 x 500 FP32 steps 203.4 ms
-// in a whole march, 198.7 with six, 197.2 with four).  Seven hides the latency
-// of short marches better where one column a thread leaves the lines few.
+// Step t loads row t + this: rows t + 3 .. are in flight.  An XCD's work-groups
+// hold that many rows of their planes in its 4 MB L2, and neighbouring chunks of
+// directions share lines there: four steps of a whole 81 x 81 x 400 x 500 FP32
+// march take 198.4 ms with seven rows ahead, 197.8 with six, 197.4 with five and
+// 197.2 with four; FP64 planes of 33 to 48 columns 5 % less with four than with
+// seven.  Seven hides the latency of short marches better (2 %) where one FP32
+// column a thread leaves the lines few.
 template <typename T, int P>
 constexpr int rows_ahead() { return sizeof(T) == 4 && P == 1 ? 7 : 4; }
 
@@ -404,8 +405,10 @@ struct MarchShape {
 // FP32: 16 directions (64-byte row segments) and one column per thread up to 64
 // columns.  From there on to 96 columns 32 directions, whole cache lines, and
 // three columns: four steps of a whole march at 81 x 81 nodes x 400 directions x
-// 500 groups 197.2 ms against 198.9 with (16, 2); alone, 81 x 21 x 121 x 500 203
-// against 261 us, 65 x 41 x 400 x 300 572 against 685.  A CU holds one such
+// 500 groups 197.2 ms against 198.9 with (16, 2), and 203.4 with that and seven
+// rows ahead, where the clipped kernel's two work-groups per CU read 7.4 GB a
+// launch for a state of 5.2, 5.6 here; alone, 81 x 21 x 121 x 500 203 against 261
+// us, 65 x 41 x 400 x 300 572 against 685.  A CU holds one such
 // work-group, so where their last round would leave much of the chip idle (81 x
 // 81 x 400 x 60, 780 of them: 327 against 300 us; 81 x 81 x 81 x 120, 360: 144
 // against 113) the smaller ones of (16, 2) are kept.  More columns per thread
