@@ -132,8 +132,9 @@ __device__ inline T limited_slope(T a, T b) {
 // accesses per cell instead of 10) whose edge steps did all of their work, one
 // kernel at a time, FP32: 9 x 9 nodes x 49 directions x 500 groups 9.8 -> 8.6
 // us, 11 x 11 x 121 x 500 24.0 -> 17.0, 13 x 13 x 81 x 500 26.6 -> 16.8, 21 x 21
-// x 400 x 500 214 -> 195 (3.6 TB/s), 81 x 81 x 400 x 250 1402 -> 1376 (3.8 TB/s);
-// FP64: 21 x 21 x 400 x 300 293 -> 198, 81 x 81 x 400 x 60 1718 -> 740.
+// x 400 x 500 214 -> 195 (3.6 TB/s), 81 x 81 x 400 x 500 2478 -> 2358 (4.5 TB/s);
+// FP64: 21 x 21 x 400 x 250 227 -> 154, 41 x 41 x 400 x 60 185 -> 164, 81 x 41 x
+// 400 x 60 929 -> 327, 97 x 41 x 400 x 60 1497 -> 749.
 enum class Part { Start, Inner, Upper, EndLoad, End };
 
 template <typename T, int MW, int P, bool CLIP>
@@ -422,8 +423,8 @@ struct MarchShape {
 // of 8 waves), 158 us for 400 x 250, against 200 with 16 (two of 6) and 170 with
 // 8; but at 13 columns (two of 5 waves against four of 4) 162 against 128 us
 // x 500.  8 directions, half lines, need the other half's work-group near: up to
-// 28 columns, or 36 where a group has few chunks (31 x 31 x 81 x 500 195 against
-// 168 us with 16, but 49 directions 86 against 107), and 49 columns and more,
+// 28 columns, or 36 where a group has few chunks (31 x 31 x 81 x 500 190 against
+// 162 us with 16, but 49 directions 84 against 101), and 49 columns and more,
 // where 16 do not fit.  Their cost counts 6 % more.  Planes above 96 columns take
 // two columns per thread.
 MarchShape march_shape(int Ny1, int nang, int Ng, size_t elem) {

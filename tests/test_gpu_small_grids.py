@@ -121,3 +121,21 @@ def test_paired_sweep_on_both_sides_of_its_limits(gpu, oracle_mod, precision, ov
             a, r = one.state(k), ref.state(k)
             np.testing.assert_array_equal(a, many.state(k))
             assert np.abs(a - r).max() <= tol * max(np.abs(r).max(), 1e-300)
+
+
+@pytest.mark.parametrize("Ng", [110, 90])  # 220 and 180 work-groups of 32 directions
+@pytest.mark.parametrize("no_clip", [0, 1])
+def test_both_arrays_of_wide_planes_in_one_launch(gpu, oracle_mod, Ng, no_clip):
+    """65 columns, with the shape of whole cache lines and with the one for fewer
+    work-groups."""
+    c = small_case(Ng=Ng, Lg=0.518 * Ng, energy=0.3 * Ng, Ny=64, Nz=2, Nmu=6, Nom=6,
+                   flags=dict(no_spatial_clipping=no_clip))
+    ref = oracle_mod.Solver(c)
+    ref.advance(3)
+    for precision, tol in ((gpu.FP64, 1e-10), (gpu.FP32, 2e-4)):
+        with gpu.Solver(c, precision) as s:
+            s.advance(3)
+            np.testing.assert_allclose(s.history()[0], ref.history()[0], rtol=tol)
+            for k in range(4):
+                a, r = s.state(k), ref.state(k)
+                assert np.abs(a - r).max() <= tol * max(np.abs(r).max(), 1e-300)
